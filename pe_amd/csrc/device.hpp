@@ -929,12 +929,13 @@ struct ConeEval {
 // of the wavefront alike, so the taken node is wave-uniform and read by the scalar unit: rounds of
 // a 6-level tree cost enough more (cross-lane reads over 64 lanes) that 20 steps in 4 rounds of 5
 // levels take 6.0k cycles against 8.2k in rounds of 6, 6, 6 and 2 (one wavefront, device libm).
+// Starts at step k0 (0 unless the first k0 steps are done: S then holds their bracket and best point).
 template <int SPEC_, class Eval>
-__device__ __forceinline__ void golden_section(GoldenState& S, int maxSub, const Eval& eval) {
+__device__ __forceinline__ void golden_section(GoldenState& S, int maxSub, const Eval& eval, int k0 = 0) {
   constexpr bool UNIFORM = SPEC_ == 6;
   constexpr int SPEC = SPEC_ == 6 ? 5 : SPEC_;
   if constexpr (SPEC == 0) {
-    for (int k = 0; k < maxSub; ++k) {
+    for (int k = k0; k < maxSub; ++k) {
       const double an = S.al + (S.ar - S.am);
       double xn0, xn1;
       const double fn = eval(an, xn0, xn1);
@@ -946,7 +947,7 @@ __device__ __forceinline__ void golden_section(GoldenState& S, int maxSub, const
     const uint32_t code = lane + 1;
     const int depth = 31 - __clz(code);   // nodes 0 .. L-2 are used: depth <= SPEC - 1
     const uint32_t base = (threadIdx.x & 63u) & ~(uint32_t)(L - 1);
-    for (int k = 0; k < maxSub; k += SPEC) {
+    for (int k = k0; k < maxSub; k += SPEC) {
       const int levels = maxSub - k < SPEC ? maxSub - k : SPEC;
       double al = S.al, ar = S.ar, am = S.am;
       bool left = S.left;
@@ -1003,6 +1004,399 @@ __device__ __forceinline__ void golden_section(GoldenState& S, int maxSub, const
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// The circle search of relaxation model 3 by a whole wavefront, with predicted outcomes.
+//
+// What bounds it is one wavefront's instruction stream (four cycles an instruction, twenty a taken
+// branch): every round of the tree search above costs a sincos, the cross-lane fold and the walk for five
+// steps.  Most outcomes are known beforehand, though, and a round that only has to check them covers up
+// to 20 steps.
+//   Isotropic tangential block (two spheres, a sphere and a plane): the energy is symmetric about the
+// bracket's centre, where its minimum lies.  The golden section then meets, every third step, two points
+// that mirror each other about the centre -- a tie: their energies differ in rounding only -- and between
+// two ties the outcomes are always "not better", "better".  A fork round evaluates every path through the
+// ties at once (two nodes a tie, constants in between); from a relaxation's second pass on, the outcomes
+// of the previous pass's ties are tried first, in one chain round.
+//   Any other block: the outcomes follow from which half of the bracket holds the energy's minimum,
+// which a few Newton steps on the circle find from the direction the bracket is centred on (or from the
+// previous pass's minimum); a chain round checks all of them.
+// Nothing rests on the predictions: every point is the one the sequential search reaches by the
+// outcomes so far, every outcome is the comparison of the energies as the sequential search evaluates
+// them, and where one was predicted wrong the search goes on without it.  So the bits are the sequential
+// search's.  On the searches of a 1,000-sphere pile, a pile of spheres, boxes and capsules and one of
+// granular particles (CPU runs), one of 459,000 isotropic searches leaves the pattern, 17 % meet a tie
+// that came out otherwise than in the pass before, and 0.5 % and 0.7 % of the others miss a prediction.
+// Measured on those searches, 20 steps on one wavefront, device libm: 6.6k cycles by tree rounds; 3.7k for an
+// isotropic search, 3.0k for one with the previous pass's ties, 3.2k for any other block.  (Correctly
+// rounded trig: 29.2k, and 14.8k and 11.3k.)  Of a 20-step chain round the walk takes 1.1k, the sincos 0.5k.
+// ---------------------------------------------------------------------------------------------
+
+// Steps a chain round covers: pe's search length (HCSITS.h:423).
+constexpr int kChainSteps = 20;
+
+// The steps of an isotropic search in threes: a tie, "not better", "better".  `r`: the tie leaves the
+// minimum in the right half of the bracket.  With p < q the two inner points at the tie, the three
+// points and the bracket after them come out the same from either side, which saves the selects that
+// step-by-step updates need: t2, t3 and the bracket [p, q] around t3, from which the next point lies left
+// exactly if r.
+struct Triple {
+  double p, q, t1, t2, t3;
+  __device__ __forceinline__ Triple(double al, double ar, double am, bool left, bool r) {
+    t1 = al + (ar - am);
+    p = left ? t1 : am;
+    q = left ? am : t1;
+    const double e1 = ar - q, e2 = q - p;
+    const double d = r ? e1 : e2, b = r ? p : al;
+    t2 = b + d;
+    const double e3 = t2 - q;
+    t3 = (r ? p : t2) + (r ? e3 : d);
+  }
+};
+
+// A node of an isotropic round: step 3 m + rem on the path whose triple j leaves the minimum right if bit
+// j of `code` is set; (al, ar, am, left): the bracket at the start of its triple.
+struct TripleNode {
+  int m, rem;
+  uint32_t code;
+  double al, ar, am;
+  bool left;
+  double an, p, q;          // the node's point, and its triple's inner points
+};
+// The bracket at the start of triple m for the lanes of triple m, all triples at once: triple j's lanes drop
+// out after j advances.  FORK: the node lanes of a fork round (triples start at lanes 0, 5, 15, 35, see
+// below); otherwise three lanes a triple.  rights: per triple j < NT - 1 the lanes whose code has bit j
+// set.  In assembly: the lanes that drop out are known, so that the execution mask is shifted (a compare
+// and a branch per advance cost 40 cycles), and the selects of all 22 instructions of an advance take
+// their masks from scalar registers.
+#define PE_TRIPLE_ADVANCE(shift, lm, rm)                                                                     \
+  "s_lshl_b64 exec, exec, " shift "\n\t"                                                                     \
+  "v_add_f64 v[8:9], v[4:5], -v[6:7]\n\t"                                                                    \
+  "v_add_f64 v[8:9], v[2:3], v[8:9]\n\t"            /* t1 */                                                 \
+  "v_cndmask_b32 v10, v6, v8, " lm "\n\t"           /* p */                                                  \
+  "v_cndmask_b32 v11, v7, v9, " lm "\n\t"                                                                    \
+  "v_cndmask_b32 v12, v8, v6, " lm "\n\t"           /* q */                                                  \
+  "v_cndmask_b32 v13, v9, v7, " lm "\n\t"                                                                    \
+  "v_add_f64 v[14:15], v[4:5], -v[12:13]\n\t"                                                                \
+  "v_add_f64 v[16:17], v[12:13], -v[10:11]\n\t"                                                              \
+  "v_cndmask_b32 v14, v16, v14, " rm "\n\t"         /* d */                                                  \
+  "v_cndmask_b32 v15, v17, v15, " rm "\n\t"                                                                  \
+  "v_cndmask_b32 v8, v2, v10, " rm "\n\t"                                                                    \
+  "v_cndmask_b32 v9, v3, v11, " rm "\n\t"                                                                    \
+  "v_add_f64 v[8:9], v[8:9], v[14:15]\n\t"          /* t2 */                                                 \
+  "v_add_f64 v[16:17], v[8:9], -v[12:13]\n\t"                                                                \
+  "v_cndmask_b32 v2, v8, v10, " rm "\n\t"                                                                    \
+  "v_cndmask_b32 v3, v9, v11, " rm "\n\t"                                                                    \
+  "v_cndmask_b32 v14, v14, v16, " rm "\n\t"                                                                  \
+  "v_cndmask_b32 v15, v15, v17, " rm "\n\t"                                                                  \
+  "v_add_f64 v[6:7], v[2:3], v[14:15]\n\t"          /* am = t3 */                                            \
+  "v_mov_b64 v[2:3], v[10:11]\n\t"                                                                           \
+  "v_mov_b64 v[4:5], v[12:13]\n\t"
+#define PE_WALK_CLOBBERS "scc", "v8", "v9", "v10", "v11", "v12", "v13", "v14", "v15", "v16", "v17"
+
+// Bit i of x in all 64 bits.
+__device__ __forceinline__ unsigned long long spread_bit(uint32_t x, int i) {
+  return (unsigned long long)((long long)((unsigned long long)x << (63 - i)) >> 63);
+}
+
+// Lanes of a fork round whose code has bit j set (code as in fork_round; the spare lanes' do not matter).
+constexpr unsigned long long fork_rights(int j) {
+  unsigned long long m = 0;
+  for (int lane = 0; lane < 64; ++lane) {
+    const int z = lane + 5, t = z >= 40 ? 3 : (z >= 20 ? 2 : (z >= 10 ? 1 : 0)), w = 1 << t, y = z - 5 * w;
+    const int code = y < w ? y : (y < 3 * w ? y - w : y - 3 * w);
+    if ((code >> j) & 1) m |= 1ull << lane;
+  }
+  return m;
+}
+
+__device__ __forceinline__ void fork_walk(double& al, double& ar, double& am, bool left) {
+  const unsigned long long l0 = spread_bit(left ? 1u : 0u, 0), r0 = fork_rights(0), r1 = fork_rights(1),
+                           r2 = fork_rights(2);
+  unsigned long long save;
+  asm volatile("s_mov_b64 %[save], exec\n\t" PE_TRIPLE_ADVANCE("5", "%[l0]", "%[r0]") PE_TRIPLE_ADVANCE("10", "%[r0]", "%[r1]")
+                   PE_TRIPLE_ADVANCE("20", "%[r1]", "%[r2]") "s_mov_b64 exec, %[save]"
+               : "+{v[2:3]}"(al), "+{v[4:5]}"(ar), "+{v[6:7]}"(am), [save] "=&s"(save)
+               : [l0] "s"(l0), [r0] "s"(r0), [r1] "s"(r1), [r2] "s"(r2)
+               : PE_WALK_CLOBBERS);
+}
+__device__ __forceinline__ void tie_walk(double& al, double& ar, double& am, uint32_t code, bool left) {
+  const unsigned long long l0 = spread_bit(left ? 1u : 0u, 0);
+  unsigned long long save;
+  asm volatile("s_mov_b64 %[save], exec\n\t" PE_TRIPLE_ADVANCE("3", "%[l0]", "%[r0]") PE_TRIPLE_ADVANCE("3", "%[r0]", "%[r1]")
+                   PE_TRIPLE_ADVANCE("3", "%[r1]", "%[r2]") PE_TRIPLE_ADVANCE("3", "%[r2]", "%[r3]")
+                       PE_TRIPLE_ADVANCE("3", "%[r3]", "%[r4]") PE_TRIPLE_ADVANCE("3", "%[r4]", "%[r5]")
+                           "s_mov_b64 exec, %[save]"
+               : "+{v[2:3]}"(al), "+{v[4:5]}"(ar), "+{v[6:7]}"(am), [save] "=&s"(save)
+               : [l0] "s"(l0), [r0] "s"(spread_bit(code, 0)), [r1] "s"(spread_bit(code, 1)),
+                 [r2] "s"(spread_bit(code, 2)), [r3] "s"(spread_bit(code, 3)), [r4] "s"(spread_bit(code, 4)),
+                 [r5] "s"(spread_bit(code, 5))
+               : PE_WALK_CLOBBERS);
+}
+template <bool FORK>
+__device__ __forceinline__ void triple_node(TripleNode& N, const GoldenState& S) {
+  N.al = S.al; N.ar = S.ar; N.am = S.am;
+  if constexpr (FORK) fork_walk(N.al, N.ar, N.am, S.left);
+  else tie_walk(N.al, N.ar, N.am, N.code, S.left);
+  N.left = N.m == 0 ? S.left : ((N.code >> (N.m - 1)) & 1u) != 0;
+  const Triple t(N.al, N.ar, N.am, N.left, ((N.code >> N.m) & 1u) != 0);
+  N.an = N.rem == 0 ? t.t1 : (N.rem == 1 ? t.t2 : t.t3);
+  N.p = t.p;
+  N.q = t.q;
+}
+// Energy and impulse of the node's point; lane 63 holds the best point so far (at the search's start, the
+// bracket's am).
+template <class Eval>
+__device__ __forceinline__ double node_energy(const TripleNode& N, const GoldenState& S, bool start, const Eval& eval,
+                                              double& x0, double& x1) {
+  const bool own = (threadIdx.x & 63u) == 63u;
+  double f = eval(own ? S.am : N.an, x0, x1);
+  if (!start && own) { f = S.fm; x0 = S.xm0; x1 = S.xm1; }
+  return f;
+}
+
+// One fork round of an isotropic search from step k (k % 3 == 0) of maxSub: 9 steps, or all the remaining
+// ones if they are at most 11 (35 and 59 nodes).  Node lanes: with z = lane + 5, triple m holds z in
+// [5, 10) * 2^m: 2^m ties, 2^(m+1) second and 2^(m+1) third steps.  False if a step left the pattern: S is
+// then as before.  The sides the ties chose are added to `code` (bit k / 3 and up).
+template <class Eval>
+__device__ __forceinline__ bool fork_round(GoldenState& S, int k, int maxSub, const Eval& eval, uint32_t& code) {
+  const int lane = (int)(threadIdx.x & 63u);
+  const int levels = maxSub - k <= 11 ? maxSub - k : 9;
+  TripleNode N;
+  const int z = lane + 5;
+  N.m = z >= 40 ? 3 : (z >= 20 ? 2 : (z >= 10 ? 1 : 0));
+  const int w = 1 << N.m, y = z - 5 * w;
+  N.rem = y < w ? 0 : (y < 3 * w ? 1 : 2);
+  N.code = (uint32_t)(y < w ? y : (y < 3 * w ? y - w : y - 3 * w));
+  triple_node<true>(N, S);
+  double x0, x1;
+  const double f = node_energy(N, S, k == 0, eval, x0, x1);
+  // the lane of the best point the sequential search holds at this node: the tie's if it was better
+  // (that is, if it changed sides against the triple before), else the previous triple's last
+  const uint32_t low = N.code & (uint32_t)(w - 1);
+  const int before = N.m == 0 ? 63 : 4 * w - 5 + (int)low, tie = 5 * w - 5 + (int)low;
+  const bool tie_better = (((N.code >> N.m) & 1u) != 0) != N.left;
+  const int src = N.rem != 0 && tie_better ? tie : before;
+  const bool lt = f < __shfl(f, src, 64);
+  const unsigned long long out = __ballot(lt);
+  uint32_t path = 0, side = S.left ? 1u : 0u;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    side ^= (uint32_t)(out >> (5 * (1 << j) - 5 + (int)path)) & 1u;
+    path |= side << j;
+  }
+  path = __builtin_amdgcn_readfirstlane(path);
+  const int step = 3 * N.m + N.rem;
+  const uint32_t codes = N.rem == 0 ? (uint32_t)(w - 1) : (uint32_t)(2 * w - 1);
+  const bool on_path = step < levels && N.code == (path & codes);
+  if (__ballot(on_path && N.rem != 0 && lt != (N.rem == 2))) return false;
+  code |= path << (k / 3);
+  if (k + levels < maxSub) {             // 9 steps: the last is better
+    const int fin = 27 + (int)(path & 7u);
+    S.al = wave_read_lane(N.p, fin);
+    S.ar = wave_read_lane(N.q, fin);
+    S.am = wave_read_lane(N.an, fin);
+    S.left = (path & 4u) != 0;
+    S.fm = wave_read_lane(f, fin);
+    S.xm0 = wave_read_lane(x0, fin);
+    S.xm1 = wave_read_lane(x1, fin);
+  } else {
+    const int fin = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__ballot(on_path && step == levels - 1)));
+    const int best = ((out >> fin) & 1ull) ? fin : __builtin_amdgcn_readlane(src, fin);
+    S.xm0 = wave_read_lane(x0, best);
+    S.xm1 = wave_read_lane(x1, best);
+  }
+  return true;
+}
+
+// One chain round of an isotropic search from its first step: all maxSub <= 20 steps, the ties' sides as in
+// `code`.  Returns the steps that came out so: if that is maxSub, S holds the result; if it is a tie's
+// place, S is the search's state there; otherwise (a step left the pattern) S is as before.
+template <class Eval>
+__device__ __forceinline__ int tie_chain(GoldenState& S, int maxSub, const Eval& eval, uint32_t code) {
+  const int lane = (int)(threadIdx.x & 63u);
+  TripleNode N;
+  N.m = lane < kChainSteps ? (lane * 11) >> 5 : 0;       // lane / 3
+  N.rem = lane < kChainSteps ? lane - 3 * N.m : 0;
+  N.code = code;
+  triple_node<false>(N, S);
+  double x0, x1;
+  const double f = node_energy(N, S, true, eval, x0, x1);
+  const bool tie_better = (((code >> N.m) & 1u) != 0) != N.left;
+  const int before = N.m == 0 ? 63 : 3 * N.m - 1;
+  const int src = N.rem != 0 && tie_better ? 3 * N.m : before;
+  const bool lt = f < __shfl(f, src, 64);
+  const bool expect = N.rem == 0 ? tie_better : N.rem == 2;
+  const uint32_t wrong = (uint32_t)__ballot(lane < maxSub && lt != expect);
+  if (!wrong) {
+    const int fin = maxSub - 1;
+    const int best = __builtin_amdgcn_readlane(expect ? lane : src, fin);
+    S.xm0 = wave_read_lane(x0, best);
+    S.xm1 = wave_read_lane(x1, best);
+    return maxSub;
+  }
+  const int at = __builtin_ctz(wrong);
+  if (at % 3 == 0) {
+    const int best = __builtin_amdgcn_readlane(src, at);
+    S.fm = wave_read_lane(f, best);
+    S.xm0 = wave_read_lane(x0, best);
+    S.xm1 = wave_read_lane(x1, best);
+    S.al = wave_read_lane(N.al, at);
+    S.ar = wave_read_lane(N.ar, at);
+    S.am = wave_read_lane(N.am, at);
+    if (at) S.left = ((code >> (at / 3 - 1)) & 1u) != 0;
+  }
+  return at;
+}
+
+// The bracket after the step to `an` with outcome lt (golden_step without the best point's values).
+__device__ __forceinline__ void golden_advance(double& al, double& ar, double& am, bool& left, double an, bool lt) {
+  const bool x = lt != left;
+  const double v = lt ? am : an;
+  al = x ? v : al;
+  ar = x ? ar : v;
+  am = lt ? an : am;
+  left = !x;
+}
+
+// Lane i's bracket after the first i < kChainSteps steps, whose outcomes are the bits of `lts`; bit i of
+// `xs`: step i moves the left end.  In assembly for the same reasons as the walks above.
+#define PE_CHAIN_STEP(i)                                                                                     \
+  "s_lshl_b64 exec, exec, 1\n\t"                                                                             \
+  "v_add_f64 v[8:9], v[4:5], -v[6:7]\n\t"                                                                    \
+  "s_bfe_i64 %[lt], %[lts], 0x10000+" #i "\n\t"                                                              \
+  "s_bfe_i64 %[x], %[xs], 0x10000+" #i "\n\t"                                                                \
+  "v_add_f64 v[8:9], v[2:3], v[8:9]\n\t"                                                                     \
+  "v_cndmask_b32 v10, v8, v6, %[lt]\n\t"                                                                     \
+  "v_cndmask_b32 v11, v9, v7, %[lt]\n\t"                                                                     \
+  "v_cndmask_b32 v2, v2, v10, %[x]\n\t"                                                                      \
+  "v_cndmask_b32 v3, v3, v11, %[x]\n\t"                                                                      \
+  "v_cndmask_b32 v4, v10, v4, %[x]\n\t"                                                                      \
+  "v_cndmask_b32 v5, v11, v5, %[x]\n\t"                                                                      \
+  "v_cndmask_b32 v6, v6, v8, %[lt]\n\t"                                                                      \
+  "v_cndmask_b32 v7, v7, v9, %[lt]\n\t"
+__device__ __forceinline__ void golden_walk(double& al, double& ar, double& am, uint32_t lts, uint32_t xs) {
+  unsigned long long lt, x, save;
+  asm volatile("s_mov_b64 %[save], exec\n\t" PE_CHAIN_STEP(0) PE_CHAIN_STEP(1) PE_CHAIN_STEP(2) PE_CHAIN_STEP(3) PE_CHAIN_STEP(4) PE_CHAIN_STEP(5)
+                   PE_CHAIN_STEP(6) PE_CHAIN_STEP(7) PE_CHAIN_STEP(8) PE_CHAIN_STEP(9) PE_CHAIN_STEP(10)
+                       PE_CHAIN_STEP(11) PE_CHAIN_STEP(12) PE_CHAIN_STEP(13) PE_CHAIN_STEP(14) PE_CHAIN_STEP(15)
+                           PE_CHAIN_STEP(16) PE_CHAIN_STEP(17) PE_CHAIN_STEP(18) "s_mov_b64 exec, %[save]"
+               : "+{v[2:3]}"(al), "+{v[4:5]}"(ar), "+{v[6:7]}"(am), [save] "=&s"(save), [lt] "=&s"(lt), [x] "=&s"(x)
+               : [lts] "s"((unsigned long long)lts), [xs] "s"((unsigned long long)xs)
+               : "scc", "v8", "v9", "v10", "v11");
+}
+
+// One chain round from the first step: min(maxSub, 20) steps with the outcomes predicted in `bits` (bit i:
+// step i better).  Returns the steps done, fewer if an outcome was predicted wrong (that step is done too,
+// with its true outcome).  A round that ends the search leaves only the best point in S.
+template <class Eval>
+__device__ __forceinline__ int chain_round(GoldenState& S, int maxSub, const Eval& eval, uint32_t bits) {
+  const int lane = (int)(threadIdx.x & 63u);
+  const int levels = maxSub < kChainSteps ? maxSub : kChainSteps;
+  // the next point lies left after an odd number of steps that were not better; x = (better != left)
+  uint32_t flips = ~bits;
+  flips ^= flips << 1; flips ^= flips << 2; flips ^= flips << 4; flips ^= flips << 8; flips ^= flips << 16;
+  const uint32_t lefts = flips << 1;      // bit i: the point of step i lies left (S.left is false)
+  double al = S.al, ar = S.ar, am = S.am;
+  golden_walk(al, ar, am, bits, bits ^ lefts);
+  const double an = lane == 63 ? S.am : al + (ar - am);
+  double x0, x1;
+  const double f = eval(an, x0, x1);
+  const uint32_t below = bits & ((1u << (lane & 31)) - 1u);
+  const int src = below ? 31 - __clz((int)below) : 63;       // the lane that evaluates this lane's am
+  const uint32_t wrong = ((uint32_t)__ballot(f < __shfl(f, src, 64)) ^ bits) & ((1u << levels) - 1u);
+  int done = levels;
+  if (wrong) {
+    done = __builtin_ctz(wrong) + 1;
+    bits ^= 1u << (done - 1);
+  }
+  bits &= (1u << done) - 1u;
+  const int best = bits ? 31 - __builtin_clz(bits) : 63;
+  S.xm0 = wave_read_lane(x0, best);
+  S.xm1 = wave_read_lane(x1, best);
+  if (done < maxSub) {
+    const int fin = done - 1;
+    S.fm = wave_read_lane(f, best);
+    S.al = wave_read_lane(al, fin);
+    S.ar = wave_read_lane(ar, fin);
+    S.am = wave_read_lane(am, fin);
+    S.left = ((lefts >> fin) & 1u) != 0;
+    golden_advance(S.al, S.ar, S.am, S.left, wave_read_lane(an, fin), ((bits >> fin) & 1u) != 0);
+  }
+  return done;
+}
+
+// What one pass's search leaves for the next one of the same relaxation.
+struct CircleMemory {
+  bool iso;                 // the tangential block is a multiple of the identity, to rounding
+  bool known = false;       // code, or at and (cs, sn), are the previous pass's
+  uint32_t code = 0;        // sides chosen at the ties
+  double at = 0, cs = 0, sn = 0;   // the energy's minimum: its angle and direction
+};
+
+// Outcomes of the first 20 steps of a search on a block that is not isotropic.
+template <class Trig>
+__device__ __forceinline__ uint32_t predict_outcomes(const GoldenState& S, const CircleEval<Trig>& ev, double centre,
+                                                     double c0, double s0, CircleMemory& M) {
+  // Newton on the circle, from the energy's derivatives over the radius in the direction (c, s)
+  double c = M.known ? M.cs : c0, s = M.known ? M.sn : s0, at = M.known ? M.at : centre;
+  const double dA = ev.flimit * (ev.A11 - ev.A00), off = ev.flimit * 0.5 * (ev.A01 + ev.A10);
+  for (int it = M.known ? 2 : 3; it > 0; --it) {
+    const double cs = c * s, c2 = fma(c, c, -(s * s));
+    const double d1 = fma(dA, cs, fma(off, c2, fma(ev.go, c, -(ev.gt * s))));
+    const double d2 = fma(dA, c2, fma(-4.0 * off, cs, -fma(ev.gt, c, ev.go * s)));
+    const double x = -d1 * __builtin_amdgcn_rcp(d2), x2 = x * x;
+    const double r = __builtin_amdgcn_rsq(1.0 + x2);
+    const double cn = fma(-x, s, c) * r;
+    s = fma(x, c, s) * r;
+    c = cn;
+    at = fma(x, fma(x2, fma(x2, 0.2, -1.0 / 3.0), 1.0), at);   // atan(x)
+  }
+  M.at = at; M.cs = c; M.sn = s;
+  // The half of the bracket that holds the minimum, step by step (u: its place in the bracket).  The next
+  // point lies in the half that the step before went to, so "better" is the same half again; the first
+  // next point lies in the right one.
+  float u = (float)((at - S.al) * __builtin_amdgcn_rcp(S.ar - S.al));
+  uint32_t right = 1;
+#pragma unroll
+  for (int i = 0; i < kChainSteps; ++i) {
+    const bool r = u > 0.5f;
+    right = right + right + (r ? 1u : 0u);
+    u = fmaf(u, 1.6180340f, r ? -0.6180340f : 0.0f);
+  }
+  return __builtin_amdgcn_readfirstlane(__brev(~(right ^ (right >> 1))) >> (32 - kChainSteps));
+}
+
+// maxSub steps of the circle search from the bracket in S (S.left false), whose best point becomes S.xm0,
+// S.xm1.  The bracket is centred on the angle `centre`, whose direction is (c0, s0).
+template <class Trig>
+__device__ __forceinline__ void golden_circle(GoldenState& S, int maxSub, const CircleEval<Trig>& ev, double centre,
+                                              double c0, double s0, CircleMemory& M) {
+  if (maxSub <= 0) return;
+  int k = 0;
+  if (M.iso) {
+    uint32_t code = 0;
+    bool on = true;
+    if (M.known) {
+      k = tie_chain(S, maxSub, ev, M.code);
+      on = k == maxSub || k % 3 == 0;
+      if (!on) k = 0;
+      code = M.code & ((1u << ((k + 2) / 3)) - 1u);
+    }
+    while (on && k < maxSub) {
+      on = fork_round(S, k, maxSub, ev, code);
+      if (on) k = maxSub - k <= 11 ? maxSub : k + 9;
+    }
+    M.code = code;
+    M.known = on && maxSub <= kChainSteps;
+  } else {
+    const uint32_t bits = predict_outcomes(S, ev, centre, c0, s0, M);
+    k = chain_round(S, maxSub, ev, bits);
+    M.known = true;
+  }
+  if (k < maxSub) golden_section<6>(S, maxSub, ev, k);
 }
 
 // One contact's NBGS update: HCSITS.h:2341-2536 (InelasticCoulombContactByDecoupling),
@@ -1237,6 +1631,9 @@ __device__ inline double relax_update(const CF& cf, const RelaxBody& b1, const R
           double c1 = 0.0, c2 = 0.0, c3 = 0.0;  // c_{j-1}, c_{j-2}, c_{j-3}
           double u1 = 0.0, u2 = 0.0;            // t_{j-2}
           double w1 = 0.0, w2 = 0.0;            // t_{j-3}
+          [[maybe_unused]] CircleMemory mem;
+          // (differences in the last bits only: D's tangential block of two spheres)
+          mem.iso = fmax(fabs(A00 - A11), fmax(fabs(A01), fabs(A10))) <= 1e-9 * A00;
           for (int j = 0; j < 20; ++j) {
             const double tq1 = pc[1], tq2 = pc[2];  // t_{j-1}
             pc[0] = 0;
@@ -1282,7 +1679,12 @@ __device__ inline double relax_update(const CF& cf, const RelaxBody& b1, const R
               const CircleEval<Trig> ev{flimit, A00, A01, A10, A11, gt, go};
               // (with SPEC > 0 the search's first round evaluates the initial point)
               if (SPEC == 0 || maxSub <= 0) gs.fm = ev(gs.am, gs.xm0, gs.xm1);
-              golden_section<SPEC>(gs, maxSub, ev);
+              if constexpr (SPEC == 6) {
+                const double rl = __builtin_amdgcn_rsq(fsq);
+                golden_circle(gs, maxSub, ev, -shift, pc[1] * rl, pc[2] * rl, mem);
+              } else {
+                golden_section<SPEC>(gs, maxSub, ev);
+              }
               pc[1] = gs.xm0;
               pc[2] = gs.xm1;
             }
