@@ -61,6 +61,10 @@ pehip_status check_params(const pehip_params* p, std::string& why);
 
 void launch_batch(int model, bool exact_trig, const Bodies& B, const RawContacts& R, const SolverContacts& C,
                   const BatchArgs& A, uint32_t grid, uint32_t threads, hipStream_t s);
+void launch_batch_fast(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C, const BatchArgs& A,
+                       uint32_t grid, uint32_t threads, hipStream_t s);
+void launch_batch_exact(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C, const BatchArgs& A,
+                        uint32_t grid, uint32_t threads, hipStream_t s);
 // queue[0] = 0, queue[1] += add_steps (a kernel, so that captured graphs hold no memset).
 void launch_batch_begin(uint32_t* queue, uint32_t add_steps, hipStream_t s);
 

@@ -1095,8 +1095,9 @@ struct TripleNode {
   "v_mov_b64 v[4:5], v[12:13]\n\t"
 #define PE_WALK_CLOBBERS "scc", "v8", "v9", "v10", "v11", "v12", "v13", "v14", "v15", "v16", "v17"
 
-// Bit i of x in all 64 bits.
+// Bit i of x, which is the same in every lane, in all 64 bits.
 __device__ __forceinline__ unsigned long long spread_bit(uint32_t x, int i) {
+  x = __builtin_amdgcn_readfirstlane(x);
   return (unsigned long long)((long long)((unsigned long long)x << (63 - i)) >> 63);
 }
 
@@ -1123,9 +1124,10 @@ __device__ __forceinline__ void fork_walk(double& al, double& ar, double& am, bo
 }
 __device__ __forceinline__ void tie_walk(double& al, double& ar, double& am, uint32_t code, bool left) {
   const unsigned long long l0 = spread_bit(left ? 1u : 0u, 0);
+  code = __builtin_amdgcn_readfirstlane(code);
   unsigned long long save;
-  asm volatile("s_mov_b64 %[save], exec\n\t" PE_TRIPLE_ADVANCE("3", "%[l0]", "%[r0]") PE_TRIPLE_ADVANCE("3", "%[r0]", "%[r1]")
-                   PE_TRIPLE_ADVANCE("3", "%[r1]", "%[r2]") PE_TRIPLE_ADVANCE("3", "%[r2]", "%[r3]")
+  asm volatile("s_mov_b64 %[save], exec\n\t" PE_TRIPLE_ADVANCE("3", "%[l0]", "%[r0]")
+                   PE_TRIPLE_ADVANCE("3", "%[r0]", "%[r1]") PE_TRIPLE_ADVANCE("3", "%[r1]", "%[r2]") PE_TRIPLE_ADVANCE("3", "%[r2]", "%[r3]")
                        PE_TRIPLE_ADVANCE("3", "%[r3]", "%[r4]") PE_TRIPLE_ADVANCE("3", "%[r4]", "%[r5]")
                            "s_mov_b64 exec, %[save]"
                : "+{v[2:3]}"(al), "+{v[4:5]}"(ar), "+{v[6:7]}"(am), [save] "=&s"(save)
@@ -1284,7 +1286,8 @@ __device__ __forceinline__ void golden_walk(double& al, double& ar, double& am, 
                        PE_CHAIN_STEP(11) PE_CHAIN_STEP(12) PE_CHAIN_STEP(13) PE_CHAIN_STEP(14) PE_CHAIN_STEP(15)
                            PE_CHAIN_STEP(16) PE_CHAIN_STEP(17) PE_CHAIN_STEP(18) "s_mov_b64 exec, %[save]"
                : "+{v[2:3]}"(al), "+{v[4:5]}"(ar), "+{v[6:7]}"(am), [save] "=&s"(save), [lt] "=&s"(lt), [x] "=&s"(x)
-               : [lts] "s"((unsigned long long)lts), [xs] "s"((unsigned long long)xs)
+               : [lts] "s"((unsigned long long)__builtin_amdgcn_readfirstlane(lts)),
+                 [xs] "s"((unsigned long long)__builtin_amdgcn_readfirstlane(xs))
                : "scc", "v8", "v9", "v10", "v11");
 }
 
@@ -1447,8 +1450,10 @@ struct GlobalFields {
 // The arithmetic of one contact's NBGS update, wherever its data live: cf(field) reads the
 // contact's fields (CF_*), b1 / b2 are its bodies, dv / dw their velocity corrections (updated in
 // place) and p its world-frame impulse (updated in place).  Returns |p_old - p_new|_inf (or
-// |p_old|_inf for a separating contact).
-template <int MODEL, class Trig, int SPEC, class CF>
+// |p_old|_inf for a separating contact).  DEFER: a contact that slides is left to the caller (kDeferred
+// is returned, and nothing the caller passed in is to be stored).
+constexpr double kDeferred = -1.0;
+template <int MODEL, class Trig, int SPEC, bool DEFER = false, class CF>
 __device__ inline double relax_update(const CF& cf, const RelaxBody& b1, const RelaxBody& b2, d3& dv1, d3& dw1,
                                       d3& dv2, d3& dw2, d3& p, int maxSub) {
   const d3 v1 = b1.v, w1 = b1.w, v2 = b2.v, w2 = b2.w;
@@ -1529,6 +1534,7 @@ __device__ inline double relax_update(const CF& cf, const RelaxBody& b1, const R
       double flimit = mu * pc[0];
       double fsq = pc[1] * pc[1] + pc[2] * pc[2];
       if (fsq > flimit * flimit || pc[0] < 0) {
+        if constexpr (DEFER) return kDeferred;
         const double dni = cf(CF_DNI);
         const double T00 = cf(CF_DTOI + 0), T01 = cf(CF_DTOI + 1);
         const double T10 = cf(CF_DTOI + 2), T11 = cf(CF_DTOI + 3);
@@ -1707,16 +1713,17 @@ __device__ inline double relax_update(const CF& cf, const RelaxBody& b1, const R
 
 // e1, e2: the contact's body entries C.b1[i], C.b2[i] (the caller has them already).
 // COHERENT: the whole wavefront owns contact i (the dataflow kernel).
-template <int MODEL, class Trig, int SPEC = 0, bool COHERENT = false>
+// DEFER: see relax_update.
+template <int MODEL, class Trig, int SPEC = 0, bool COHERENT = false, bool DEFER = false>
 __device__ inline double relax_contact(const SolverContacts& C, size_t i, uint32_t e1, uint32_t e2,
                                        const double* __restrict__ sb, double* __restrict__ dvw, double dtinv,
                                        int maxSub);
-template <int MODEL, class Trig, int SPEC = 0, bool COHERENT = false>
+template <int MODEL, class Trig, int SPEC = 0, bool COHERENT = false, bool DEFER = false>
 __device__ inline double relax_contact(const SolverContacts& C, size_t i, const double* __restrict__ sb,
                                        double* __restrict__ dvw, double dtinv, int maxSub) {
-  return relax_contact<MODEL, Trig, SPEC, COHERENT>(C, i, C.b1[i], C.b2[i], sb, dvw, dtinv, maxSub);
+  return relax_contact<MODEL, Trig, SPEC, COHERENT, DEFER>(C, i, C.b1[i], C.b2[i], sb, dvw, dtinv, maxSub);
 }
-template <int MODEL, class Trig, int SPEC, bool COHERENT>
+template <int MODEL, class Trig, int SPEC, bool COHERENT, bool DEFER>
 __device__ inline double relax_contact(const SolverContacts& C, size_t i, uint32_t e1, uint32_t e2,
                                        const double* __restrict__ sb, double* __restrict__ dvw, double dtinv,
                                        int maxSub) {
@@ -1750,7 +1757,8 @@ __device__ inline double relax_contact(const SolverContacts& C, size_t i, uint32
     p = mk3(f[CF_P * cap + i], f[(CF_P + 1) * cap + i], f[(CF_P + 2) * cap + i]);
   }
   const GlobalFields cf{f, cap, i};
-  const double delta = relax_update<MODEL, Trig, SPEC>(cf, B1, B2, dv1, dw1, dv2, dw2, p, maxSub);
+  const double delta = relax_update<MODEL, Trig, SPEC, DEFER>(cf, B1, B2, dv1, dw1, dv2, dw2, p, maxSub);
+  if (DEFER && delta == kDeferred) return delta;
   // one lane of the contact's group stores (COHERENT: the whole wavefront owns the contact)
   const uint32_t group_mask = COHERENT ? 63u : ((1u << SPEC) - 1u);
   if ((threadIdx.x & group_mask) == 0) {
