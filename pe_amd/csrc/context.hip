@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "context.hpp"
+#include "resident.hpp"
 
 using namespace pe_amd;
 
@@ -25,11 +26,21 @@ constexpr uint32_t kDataflowMaxContacts = 65536;
 constexpr uint32_t kDataflowSpinLimit = 1u << 22;
 // With an abort threshold the host reads the device's stop flag once per this many sweeps.
 constexpr uint32_t kAbortPoll = 32;
-// Automatic schedule with an abort threshold: one workgroup runs all sweeps up to this many
-// contacts (relaxation models 0 and 1: one pass of its 512 lanes per colour), where a colour
-// launch is mostly launch latency.  Beyond it the workgroup needs several passes per colour and
-// the colour launches are faster.
-constexpr uint32_t kSingleBlockMaxContacts = 512;
+// Automatic schedule: one workgroup runs all sweeps of a step while it holds all the contacts on the chip
+// (models without a search), or up to a few contacts (models with one).  A colour costs it 1 to 2 us; an
+// update costs the dataflow sweeps about 4 us, and so does a colour launch, the choice with an abort
+// threshold.  But it relaxes only four sliding contacts at a time.  50 sweeps, one workgroup against
+// dataflow: model 1 0.22 against 0.41 ms (18 contacts), 0.22 against 0.65 (100), 0.23 against 0.63 (194), 0.43
+// against 0.66 (281), 0.48 against 0.70 (408); model 3 0.17 against 0.27 (5), 0.44 against 0.50 (18), 0.96
+// against 0.79 (39), 3.2 against 1.0 (144).
+constexpr uint32_t kSingleBlockMaxContacts = kResidentWide, kSingleBlockMaxSearching = 16;
+
+bool is_searching(int model) { return model == PEHIP_INELASTIC_COULOMB_DECOUPLING || model == PEHIP_INELASTIC_GMD; }
+
+// The automatic schedule's choice of one workgroup for a step of nc contacts.
+bool choose_single_block(const pehip_params& P, uint32_t nc) {
+  return nc <= (is_searching(P.relaxation_model) ? kSingleBlockMaxSearching : kSingleBlockMaxContacts);
+}
 std::string g_create_error;
 
 uint32_t next_pow2(uint64_t x) {
@@ -824,9 +835,7 @@ pehip_status pe_one_step(pehip_ctx* ctx, double dt) {
       CKS(sync_check(ctx));
       iters = (uint32_t)(*(unsigned long long*)ctx->hstage);
     } else if (P.sweep_schedule == PEHIP_SCHEDULE_SINGLE_BLOCK ||
-               (P.sweep_schedule == PEHIP_SCHEDULE_AUTO && P.abort_threshold > 0 &&
-                P.relaxation_model != PEHIP_INELASTIC_COULOMB_DECOUPLING &&
-                P.relaxation_model != PEHIP_INELASTIC_GMD && nc <= kSingleBlockMaxContacts)) {
+               (P.sweep_schedule == PEHIP_SCHEDULE_AUTO && choose_single_block(P, nc))) {
       ColourOffsets O;
       O.ncol = (uint32_t)ctx->colour_off.size() - 1;
       for (uint32_t k = 0; k <= O.ncol; ++k) O.off[k] = ctx->colour_off[k];
@@ -835,9 +844,12 @@ pehip_status pe_one_step(pehip_ctx* ctx, double dt) {
                          (int)P.max_sub_iterations, P.abort_threshold, ctx->deltas, s);
       if (ctx->profiling) CKS(record_launch_event(ctx, 1));
       ctx->n_launch_events = ctx->profiling ? 2 : 0;
-      CK(hipMemcpyAsync(ctx->hstage, ctx->deltas + P.max_iterations, 8, hipMemcpyDeviceToHost, s));
-      CKS(sync_check(ctx));
-      iters = (uint32_t)(*(unsigned long long*)ctx->hstage);
+      iters = P.max_iterations;
+      if (P.abort_threshold > 0) {
+        CK(hipMemcpyAsync(ctx->hstage, ctx->deltas + P.max_iterations, 8, hipMemcpyDeviceToHost, s));
+        CKS(sync_check(ctx));
+        iters = (uint32_t)(*(unsigned long long*)ctx->hstage);
+      }
       schedule_used = PEHIP_SCHEDULE_SINGLE_BLOCK;
     } else {
       // All sweeps in one cooperative launch (same Gauss-Seidel order per body as the colours).

@@ -1,6 +1,7 @@
 // Solver kernels: contact-graph colouring, contact caching and the NBGS sweeps.
 #include <algorithm>
 
+#include "resident.hpp"
 #include "step_ops.hpp"
 
 namespace pe_amd {
@@ -184,6 +185,103 @@ __global__ void __launch_bounds__(256) k_sweep(SolverContacts C, uint32_t begin,
   wave_max_atomic(d, delta);
 }
 
+// All sweeps of a step in one workgroup, its contacts on the chip (see resident.hpp): for steps of at most
+// THREADS contacts.  As k_sweep_block otherwise, except that only the sweeps an abort test looks at,
+// and the last one, leave their impulse change.
+template <int MODEL, class Trig, uint32_t THREADS>
+__global__ void __launch_bounds__(THREADS) k_sweep_resident(SolverContacts C, ColourOffsets O, uint32_t iters,
+                                                            const double* sb, double* dvw, int maxSub, double thr,
+                                                            unsigned long long* deltas) {
+  constexpr bool kHold = THREADS == kResidentThreads;
+  // open-addressing table of the non-fixed bodies, at most 2 * THREADS
+  constexpr uint32_t kTable = kHold ? 1024 : 2048;
+  static_assert(kTable > 2 * THREADS, "the table keeps a free place");
+  __shared__ uint32_t body[kTable];
+  __shared__ double ldvw[6 * kTable];
+  __shared__ unsigned long long wmax[THREADS / 64];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t nc = O.off[O.ncol];
+  for (uint32_t i = tid; i < kTable; i += THREADS) body[i] = kNoBody;
+  __syncthreads();
+  // With a search a colour's slots, which follow one another, are spread over the wavefronts, which relax
+  // their sliding contacts one by one; without, they stay together, so that the other wavefronts pass a
+  // colour by (72 contacts of a colour in all of 12 wavefronts: 7 us a colour).
+  const uint32_t slot = MODEL == 3 || MODEL == 5 ? lane * (THREADS / 64) + wave : tid;
+  const bool have = slot < nc;
+  uint32_t colour = kMaxColours;
+  auto place = [&](uint32_t b) {
+    uint32_t h = mix32(b) & (kTable - 1);
+    for (;;) {                       // (the table always has a free place)
+      const uint32_t old = atomicCAS(&body[h], kNoBody, b);
+      if (old == kNoBody || old == b) return h;
+      h = (h + 1) & (kTable - 1);
+    }
+  };
+  ResidentContact<kHold> r;
+  if (have) {
+    resident_load(r, C, slot, sb, place);
+    for (colour = 0; slot >= O.off[colour + 1]; ++colour) {}
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < kTable; i += THREADS)
+    if (body[i] != kNoBody)
+      for (uint32_t k = 0; k < 6; ++k) ldvw[6 * i + k] = dvw[(size_t)kDVW * body[i] + k];
+  __syncthreads();
+  uint32_t it = 0;
+  while (it < iters) {
+    // non-negative doubles (and NaN above +inf) order like their bit patterns
+    unsigned long long u = 0;
+    for (uint32_t k = 0; k < O.ncol; ++k) {
+      const unsigned long long d =
+          (unsigned long long)__double_as_longlong(resident_relax<MODEL, Trig, kHold>(r, colour == k, ldvw, maxSub));
+      u = d > u ? d : u;
+      __syncthreads();
+    }
+    ++it;
+    if (thr > 0 || it == iters) {
+#pragma unroll
+      for (int x = 32; x > 0; x >>= 1) {
+        const unsigned long long o = __shfl_xor(u, x, 64);
+        u = o > u ? o : u;
+      }
+      if (lane == 0) wmax[wave] = u;
+      __syncthreads();
+      unsigned long long m = 0;
+      for (uint32_t w = 0; w < THREADS / 64; ++w) m = wmax[w] > m ? wmax[w] : m;
+      __syncthreads();
+      if (tid == 0) deltas[it - 1] = m;
+      if (thr > 0 && __longlong_as_double((long long)m) < thr) break;
+    }
+  }
+  if (tid == 0) deltas[iters] = it;
+  if (have) {
+    C.f[CF_P * C.cap + slot] = r.p.x;
+    C.f[(CF_P + 1) * C.cap + slot] = r.p.y;
+    C.f[(CF_P + 2) * C.cap + slot] = r.p.z;
+  }
+  for (uint32_t i = tid; i < kTable; i += THREADS)
+    if (body[i] != kNoBody)
+      for (uint32_t k = 0; k < 6; ++k) dvw[(size_t)kDVW * body[i] + k] = ldvw[6 * i + k];
+}
+
+template <class Trig>
+static void resident_dispatch(int model, const SolverContacts& C, const ColourOffsets& O, uint32_t iters,
+                              const Bodies& B, int maxSub, double thr, unsigned long long* deltas, hipStream_t s) {
+  const bool wide = O.off[O.ncol] > kResidentThreads;
+  const dim3 g(1), b(wide ? kResidentWide : kResidentThreads);
+#define PE_RESIDENT(model, threads) \
+  hipLaunchKernelGGL((k_sweep_resident<model, Trig, threads>), g, b, 0, s, C, O, iters, B.sb, B.dvw, maxSub, thr, deltas)
+  switch (model) {
+    case 0: if (wide) PE_RESIDENT(0, kResidentWide); else PE_RESIDENT(0, kResidentThreads); break;
+    case 1: if (wide) PE_RESIDENT(1, kResidentWide); else PE_RESIDENT(1, kResidentThreads); break;
+    case 2: if (wide) PE_RESIDENT(2, kResidentWide); else PE_RESIDENT(2, kResidentThreads); break;
+    case 4: if (wide) PE_RESIDENT(4, kResidentWide); else PE_RESIDENT(4, kResidentThreads); break;
+    case 5: PE_RESIDENT(5, kResidentThreads); break;
+    default: PE_RESIDENT(3, kResidentThreads); break;
+  }
+#undef PE_RESIDENT
+}
+
 // All sweeps of a step in one workgroup: colour k's contacts are spread over the workgroup's
 // groups of 2^SPEC lanes, a barrier separates colours (the contacts of one colour share no
 // non-fixed body, so this is the colour launches' computation, bit for bit), and the abort test
@@ -249,6 +347,12 @@ static void block_dispatch(int model, const SolverContacts& C, const ColourOffse
 void launch_sweep_block(int model, bool exact_trig, const SolverContacts& C, const ColourOffsets& O, uint32_t iters,
                         const Bodies& B, double dtinv, int maxSub, double thr, unsigned long long* deltas,
                         hipStream_t s) {
+  const bool searches = model == 3 || model == 5;
+  if (O.off[O.ncol] <= (searches ? kResidentThreads : kResidentWide)) {
+    if (exact_trig) resident_dispatch<TrigExact>(model, C, O, iters, B, maxSub, thr, deltas, s);
+    else resident_dispatch<TrigFast>(model, C, O, iters, B, maxSub, thr, deltas, s);
+    return;
+  }
   if (exact_trig) block_dispatch<TrigExact>(model, C, O, iters, B, dtinv, maxSub, thr, deltas, s);
   else block_dispatch<TrigFast>(model, C, O, iters, B, dtinv, maxSub, thr, deltas, s);
 }
