@@ -39,7 +39,7 @@ struct AdjointState {
   // reverse-pass work space
   std::vector<StepTape> tape;
   uint32_t ccap = 0;
-  double *jac = nullptr, *minv = nullptr, *lambda = nullptr, *alpha = nullptr;
+  double *jac = nullptr, *pk = nullptr, *lambda = nullptr, *alpha = nullptr;
   double *xbar = nullptr, *vbar = nullptr, *wbar = nullptr, *mubar = nullptr;
   unsigned long long* delta = nullptr;
 };
@@ -56,7 +56,7 @@ void pe_adjoint_free(pehip_ctx* ctx) {
   for (auto& c : a->checkpoints) dfree(c);
   dfree(a->final_state);
   for (auto& t : a->tape) free_tape(t);
-  dfree(a->jac); dfree(a->minv); dfree(a->lambda); dfree(a->alpha);
+  dfree(a->jac); dfree(a->pk); dfree(a->lambda); dfree(a->alpha);
   dfree(a->xbar); dfree(a->vbar); dfree(a->wbar); dfree(a->mubar); dfree(a->delta);
   delete a;
   ctx->adj = nullptr;
@@ -127,11 +127,11 @@ static pehip_status record(pehip_ctx* ctx, AdjointState* a, StepTape& t, const d
     adj_pack_p(nc, ctx->sol.f, ctx->sol.cap, t.p, t.mu, s);
   }
   if (nc > a->ccap) {
-    dfree(a->jac); dfree(a->minv); dfree(a->lambda);
+    dfree(a->jac); dfree(a->pk); dfree(a->lambda);
     a->ccap = 0;
     const uint32_t cap = std::max<uint32_t>(nc + nc / 4, 1024);
     CK(dalloc(a->jac, (size_t)cap * ad::kAdjIn * ad::kAdjOut));
-    CK(dalloc(a->minv, 9 * (size_t)cap));
+    CK(dalloc(a->pk, (size_t)kAdjSweepFields * cap));
     CK(dalloc(a->lambda, 3 * (size_t)cap));
     a->ccap = cap;
   }
@@ -151,12 +151,22 @@ static pehip_status reverse_step(pehip_ctx* ctx, AdjointState* a, const StepTape
   if (t.nc) {
     fill_u64((unsigned long long*)a->lambda, 0ull, 3 * (size_t)t.nc, s);
     adj_jacobian(a->prm.relaxation_model, T, A, a->jac, s);
-    adj_prepare(t.nc, a->jac, a->minv, s);
+    adj_prepare(t.nc, a->jac, a->pk, s);
     const uint32_t ncol = (uint32_t)t.colour_off.size() - 1;
-    for (uint32_t it = 0; it < sweeps; ++it) {
+    ColourOffsets O;
+    O.ncol = ncol;
+    for (uint32_t k = 0; k <= ncol; ++k) O.off[k] = t.colour_off[k];
+    const bool in_block = adj_block(T, O, n, a->pk, a->alpha, a->lambda, sweeps, tol, a->delta, s);
+    if (in_block) {
+      CK(hipMemcpyAsync(ctx->hstage, a->delta, 16, hipMemcpyDeviceToHost, s));
+      CKS(sync_check(ctx));
+      *used = (uint32_t)(*(unsigned long long*)ctx->hstage);
+      std::memcpy(last_delta, ctx->hstage + 2, 8);
+    }
+    for (uint32_t it = 0; it < sweeps && !in_block; ++it) {
       fill_u64(a->delta, 0ull, 1, s);
       for (uint32_t k = 0; k < ncol; ++k)
-        adj_sweep(T, t.colour_off[k], t.colour_off[k + 1], a->jac, a->minv, a->alpha, a->lambda, a->delta, s);
+        adj_sweep(T, t.colour_off[k], t.colour_off[k + 1], a->pk, a->alpha, a->lambda, a->delta, s);
       *used = it + 1;
       if (tol > 0 && (it % 8 == 7 || it + 1 == sweeps)) {
         CK(hipMemcpyAsync(ctx->hstage, a->delta, 8, hipMemcpyDeviceToHost, s));
@@ -165,7 +175,7 @@ static pehip_status reverse_step(pehip_ctx* ctx, AdjointState* a, const StepTape
         if (*last_delta < tol) break;
       }
     }
-    if (tol <= 0) {
+    if (tol <= 0 && !in_block) {
       CK(hipMemcpyAsync(ctx->hstage, a->delta, 8, hipMemcpyDeviceToHost, s));
       CKS(sync_check(ctx));
       std::memcpy(last_delta, ctx->hstage, 8);
@@ -228,7 +238,7 @@ pehip_status pehip_adjoint_backward(pehip_ctx* ctx, const double* dL_dpos, const
   if (!a->wbar) CK(dalloc(a->wbar, 3 * n));
   if (!a->alpha) CK(dalloc(a->alpha, 6 * n));
   if (!a->mubar) CK(dalloc(a->mubar, 1));
-  if (!a->delta) CK(dalloc(a->delta, 1));
+  if (!a->delta) CK(dalloc(a->delta, 2));
   fill_u64((unsigned long long*)a->xbar, 0ull, 3 * n, s);
   fill_u64((unsigned long long*)a->vbar, 0ull, 3 * n, s);
   fill_u64((unsigned long long*)a->wbar, 0ull, 3 * n, s);

@@ -414,11 +414,17 @@ struct AdjConsts {
 };
 
 void adj_jacobian(int model, const AdjTape& T, const AdjConsts& A, double* jac, hipStream_t s);
-void adj_prepare(uint32_t nc, const double* jac, double* minv, hipStream_t s);
+// Doubles per contact that an adjoint sweep reads (written by adj_prepare, field-major).
+constexpr int kAdjSweepFields = 81;
+void adj_prepare(uint32_t nc, const double* jac, double* pk, hipStream_t s);
 void adj_init(uint32_t n, const uint8_t* fixed, const double* xbar, const double* vbar, const double* wbar, double dt,
               double* alpha, hipStream_t s);
-void adj_sweep(const AdjTape& T, uint32_t begin, uint32_t end, const double* jac, const double* minv, double* alpha,
-               double* lambda, unsigned long long* delta, hipStream_t s);
+void adj_sweep(const AdjTape& T, uint32_t begin, uint32_t end, const double* pk, double* alpha, double* lambda,
+               unsigned long long* delta, hipStream_t s);
+// All sweeps in one workgroup (see k_adj_block), for up to kAdjBlockContacts contacts; false beyond.
+constexpr uint32_t kAdjHeldContacts = 512, kAdjHeldBodies = 2048, kAdjBlockContacts = 2048;
+bool adj_block(const AdjTape& T, const struct ColourOffsets& O, uint32_t n, const double* pk, double* alpha,
+               double* lambda, uint32_t sweeps, double tol, unsigned long long* out, hipStream_t s);
 void adj_assemble(const AdjTape& T, const double* jac, const double* alpha, const double* lambda, double* xbar,
                   double* mubar, hipStream_t s);
 void adj_finish(uint32_t n, const double* alpha, double* vbar, double* wbar, hipStream_t s);

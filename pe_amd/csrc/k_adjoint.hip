@@ -4,9 +4,11 @@
 // the start of the step, solver body records, post-solve velocities):
 //   k_adj_jacobian  one thread per (contact, input direction): contact_map() in dual numbers
 //                   gives one column of the contact's 15 x 22 Jacobian;
-//   k_adj_prepare   per contact, the 3 x 3 matrix of the transposed local system and its inverse;
+//   k_adj_prepare   per contact, what a sweep reads: the Jacobian's velocity and impulse blocks and the
+//                   inverse of the transposed local system's 3 x 3 matrix, field-major;
 //   k_adj_init      body adjoints alpha = adjoint of the post-solve velocities;
 //   k_adj_sweep     one colour of a Gauss-Seidel sweep on the transposed (adjoint) system;
+//   k_adj_block     all sweeps of a step in one workgroup, for few contacts;
 //   k_adj_assemble  position and friction adjoints from the converged (alpha, lambda).
 #include "adjoint.hpp"
 #include "kernels.hpp"
@@ -82,7 +84,10 @@ __device__ __forceinline__ double jget(const double* jac, uint32_t s, int j, int
 }
 
 // Mc = P_p^T - Q_p^T P_U^T (P_p = dE2/dp, Q_p = d(-contrib)/dp, P_U = dE2/dU), inverted.
-__global__ void k_adj_prepare(uint32_t nc, const double* jac, double* minv) {
+// Fields of a contact in `pk` (field f of contact s at pk[f * nc + s]): P_U^T, 12 x 3; Q_p^T, 3 x 12; Mc^-1.
+constexpr int AK_PU = 0, AK_QP = 36, AK_MI = 72;
+static_assert(AK_MI + 9 == kAdjSweepFields, "fields of a contact in an adjoint sweep");
+__global__ void k_adj_prepare(uint32_t nc, const double* jac, double* pk) {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nc) return;
   m33 M;
@@ -95,8 +100,13 @@ __global__ void k_adj_prepare(uint32_t nc, const double* jac, double* minv) {
       M.a[3 * a + b] = v;
     }
   const m33 Mi = mat_inv(M);
+  for (int m = 0; m < 12; ++m)
+    for (int c = 0; c < 3; ++c) {
+      pk[(size_t)(AK_PU + 3 * m + c) * nc + s] = jget(jac, s, 6 + m, c);
+      pk[(size_t)(AK_QP + 12 * c + m) * nc + s] = jget(jac, s, 18 + c, 3 + m);
+    }
 #pragma unroll
-  for (int k = 0; k < 9; ++k) minv[9 * (size_t)s + k] = Mi.a[k];
+  for (int k = 0; k < 9; ++k) pk[(size_t)(AK_MI + k) * nc + s] = Mi.a[k];
 }
 
 // alpha_b = (vbar + dt * xbar, wbar) for non-fixed bodies, 0 for fixed ones.
@@ -127,54 +137,162 @@ __device__ __forceinline__ void wave_max_u64(double v, unsigned long long* out) 
   if ((threadIdx.x & 63) == 0 && u) atomicMax(out, u);
 }
 
+// One contact's update of an adjoint sweep: f(k) reads its fields, a1 / a2 are its non-fixed bodies'
+// adjoints (null for fixed ones) and l its lambda, updated in place.  Returns the largest change of lambda.
+template <class F>
+__device__ __forceinline__ double adj_relax(const F& f, double* a1, double* a2, double* l) {
+  double a[12];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    a[k] = a1 ? a1[k] : 0.0;
+    a[6 + k] = a2 ? a2[k] : 0.0;
+  }
+  double ln[3];
+  // remove the contact's own term: a += P_U^T lambda_old
+#pragma unroll
+  for (int m = 0; m < 12; ++m)
+    a[m] += f(AK_PU + 3 * m) * l[0] + f(AK_PU + 3 * m + 1) * l[1] + f(AK_PU + 3 * m + 2) * l[2];
+  double rhs[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    double v = 0.0;
+#pragma unroll
+    for (int m = 0; m < 12; ++m) v -= f(AK_QP + 12 * c + m) * a[m];
+    rhs[c] = v;
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    ln[c] = f(AK_MI + 3 * c) * rhs[0] + f(AK_MI + 3 * c + 1) * rhs[1] + f(AK_MI + 3 * c + 2) * rhs[2];
+#pragma unroll
+  for (int m = 0; m < 12; ++m)
+    a[m] -= f(AK_PU + 3 * m) * ln[0] + f(AK_PU + 3 * m + 1) * ln[1] + f(AK_PU + 3 * m + 2) * ln[2];
+  if (a1)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) a1[k] = a[k];
+  if (a2)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) a2[k] = a[6 + k];
+  double d = 0.0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    d = fmax(d, fabs(ln[k] - l[k]));
+    l[k] = ln[k];
+  }
+  return d;
+}
+
+struct AdjFields {
+  const double* pk;
+  size_t nc, s;
+  __device__ __forceinline__ double operator()(int k) const { return pk[(size_t)k * nc + s]; }
+};
+struct AdjHeldFields {
+  double v[kAdjSweepFields];
+  __device__ __forceinline__ double operator()(int k) const { return v[k]; }
+};
+
 // One colour of the adjoint sweep: contacts [begin, end) share no non-fixed body.
-__global__ void k_adj_sweep(AdjTape T, uint32_t begin, uint32_t end, const double* jac, const double* minv,
-                            double* alpha, double* lambda, unsigned long long* delta) {
+__global__ void k_adj_sweep(AdjTape T, uint32_t begin, uint32_t end, const double* pk, double* alpha, double* lambda,
+                            unsigned long long* delta) {
   const uint32_t s = begin + blockIdx.x * blockDim.x + threadIdx.x;
   double d = 0.0;
   if (s < end) {
     const uint32_t e1 = T.b1[s], e2 = T.b2[s];
-    const uint32_t i1 = e1 & ~kFixedBit, i2 = e2 & ~kFixedBit;
-    const bool f1 = (e1 & kFixedBit) != 0, f2 = (e2 & kFixedBit) != 0;
-    double a[12];
+    double l[3];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      a[k] = f1 ? 0.0 : alpha[6 * (size_t)i1 + k];
-      a[6 + k] = f2 ? 0.0 : alpha[6 * (size_t)i2 + k];
-    }
-    double lo[3], ln[3];
+    for (int k = 0; k < 3; ++k) l[k] = lambda[3 * (size_t)s + k];
+    d = adj_relax(AdjFields{pk, T.nc, s}, (e1 & kFixedBit) ? nullptr : alpha + 6 * (size_t)e1,
+                  (e2 & kFixedBit) ? nullptr : alpha + 6 * (size_t)e2, l);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) lo[k] = lambda[3 * (size_t)s + k];
-    // remove the contact's own term: a += P_U^T lambda_old
-#pragma unroll
-    for (int m = 0; m < 12; ++m)
-      a[m] += jget(jac, s, 6 + m, 0) * lo[0] + jget(jac, s, 6 + m, 1) * lo[1] + jget(jac, s, 6 + m, 2) * lo[2];
-    double rhs[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      double v = 0.0;
-      for (int m = 0; m < 12; ++m) v -= jget(jac, s, 18 + c, 3 + m) * a[m];
-      rhs[c] = v;
-    }
-    const double* Mi = minv + 9 * (size_t)s;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) ln[c] = Mi[3 * c] * rhs[0] + Mi[3 * c + 1] * rhs[1] + Mi[3 * c + 2] * rhs[2];
-#pragma unroll
-    for (int m = 0; m < 12; ++m)
-      a[m] -= jget(jac, s, 6 + m, 0) * ln[0] + jget(jac, s, 6 + m, 1) * ln[1] + jget(jac, s, 6 + m, 2) * ln[2];
-    if (!f1)
-#pragma unroll
-      for (int k = 0; k < 6; ++k) alpha[6 * (size_t)i1 + k] = a[k];
-    if (!f2)
-#pragma unroll
-      for (int k = 0; k < 6; ++k) alpha[6 * (size_t)i2 + k] = a[6 + k];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      lambda[3 * (size_t)s + k] = ln[k];
-      d = fmax(d, fabs(ln[k] - lo[k]));
-    }
+    for (int k = 0; k < 3; ++k) lambda[3 * (size_t)s + k] = l[k];
   }
   wave_max_u64(d, delta);
+}
+
+// All sweeps of a step in one workgroup, a barrier between colours (the contacts of one share no non-fixed
+// body, so these are the colour launches' updates, bit for bit) and the host's test for the end -- the
+// change of every eighth sweep and of the last against tol, if tol > 0.  out[0]: sweeps done, out[1]: the
+// change last looked at (the last sweep's without tol).
+//
+// What bounds it is the latency of a colour.  HOLD: one contact a thread with its 81 fields in registers for
+// all sweeps and the adjoints of all bodies in LDS (kAdjHeldBodies); otherwise fields and adjoints come from
+// L2.  576 contacts in 8 colours, 2,000 sweeps: about 45 ms from L2 against 130 by colour launches (1,024
+// threads, whose 128 registers do not hold a contact's fields at once: 117); up to 180 contacts in 2 or 3
+// colours, held: 2.2 us a sweep against 12.
+template <bool HOLD, uint32_t THREADS>
+__global__ void __launch_bounds__(THREADS) k_adj_block(AdjTape T, ColourOffsets O, uint32_t n, const double* pk,
+                                                       double* alpha, double* lambda, uint32_t sweeps, double tol,
+                                                       unsigned long long* out) {
+  __shared__ double la[HOLD ? 6 * kAdjHeldBodies : 1];
+  __shared__ unsigned long long wmax[THREADS / 64];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  AdjHeldFields held;
+  double hl[3];
+  double *h1 = nullptr, *h2 = nullptr;
+  uint32_t colour = kMaxColours;
+  if constexpr (HOLD) {
+    for (uint32_t i = tid; i < 6 * n; i += THREADS) la[i] = alpha[i];
+    if (tid < T.nc) {
+#pragma unroll
+      for (int k = 0; k < kAdjSweepFields; ++k) held.v[k] = pk[(size_t)k * T.nc + tid];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) hl[k] = lambda[3 * (size_t)tid + k];
+      const uint32_t e1 = T.b1[tid], e2 = T.b2[tid];
+      h1 = (e1 & kFixedBit) ? nullptr : la + 6 * e1;
+      h2 = (e2 & kFixedBit) ? nullptr : la + 6 * e2;
+      for (colour = 0; tid >= O.off[colour + 1]; ++colour) {}
+    }
+    __syncthreads();
+  }
+  uint32_t it = 0;
+  unsigned long long seen = 0;
+  while (it < sweeps) {
+    // non-negative doubles order like their bit patterns
+    unsigned long long u = 0;
+    for (uint32_t k = 0; k < O.ncol; ++k) {
+      if constexpr (HOLD) {
+        if (colour == k) u = (unsigned long long)__double_as_longlong(adj_relax(held, h1, h2, hl));
+      } else {
+        for (uint32_t s = O.off[k] + tid; s < O.off[k + 1]; s += THREADS) {
+          const uint32_t e1 = T.b1[s], e2 = T.b2[s];
+          double l[3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) l[c] = lambda[3 * (size_t)s + c];
+          const unsigned long long d = (unsigned long long)__double_as_longlong(
+              adj_relax(AdjFields{pk, T.nc, s}, (e1 & kFixedBit) ? nullptr : alpha + 6 * (size_t)e1,
+                        (e2 & kFixedBit) ? nullptr : alpha + 6 * (size_t)e2, l));
+#pragma unroll
+          for (int c = 0; c < 3; ++c) lambda[3 * (size_t)s + c] = l[c];
+          u = d > u ? d : u;
+        }
+      }
+      __syncthreads();
+    }
+    ++it;
+    if (it == sweeps || (tol > 0 && it % 8 == 0)) {
+#pragma unroll
+      for (int x = 32; x > 0; x >>= 1) {
+        const unsigned long long o = __shfl_xor(u, x, 64);
+        u = o > u ? o : u;
+      }
+      if (lane == 0) wmax[wave] = u;
+      __syncthreads();
+      seen = 0;
+      for (uint32_t w = 0; w < THREADS / 64; ++w) seen = wmax[w] > seen ? wmax[w] : seen;
+      __syncthreads();
+      if (tol > 0 && __longlong_as_double((long long)seen) < tol) break;
+    }
+  }
+  if constexpr (HOLD) {
+    for (uint32_t i = tid; i < 6 * n; i += THREADS) alpha[i] = la[i];
+    if (tid < T.nc)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) lambda[3 * (size_t)tid + k] = hl[k];
+  }
+  if (tid == 0) {
+    out[0] = it;
+    out[1] = seen;
+  }
 }
 
 // xbar += -(Q_x^T alpha_c + P_x^T lambda_c) per contact; mubar += -P_mu . lambda.
@@ -266,18 +384,28 @@ void adj_jacobian(int model, const AdjTape& T, const AdjConsts& A, double* jac, 
   else if (model == 1) hipLaunchKernelGGL(k_adj_jacobian<1>, blocks(n), dim3(256), 0, s, T, A, jac);
   else hipLaunchKernelGGL(k_adj_jacobian<3>, blocks(n), dim3(256), 0, s, T, A, jac);
 }
-void adj_prepare(uint32_t nc, const double* jac, double* minv, hipStream_t s) {
-  if (nc) hipLaunchKernelGGL(k_adj_prepare, blocks(nc), dim3(256), 0, s, nc, jac, minv);
+void adj_prepare(uint32_t nc, const double* jac, double* pk, hipStream_t s) {
+  if (nc) hipLaunchKernelGGL(k_adj_prepare, blocks(nc), dim3(256), 0, s, nc, jac, pk);
 }
 void adj_init(uint32_t n, const uint8_t* fixed, const double* xbar, const double* vbar, const double* wbar, double dt,
               double* alpha, hipStream_t s) {
   hipLaunchKernelGGL(k_adj_init, blocks(n), dim3(256), 0, s, n, fixed, xbar, vbar, wbar, dt, alpha);
 }
-void adj_sweep(const AdjTape& T, uint32_t begin, uint32_t end, const double* jac, const double* minv, double* alpha,
-               double* lambda, unsigned long long* delta, hipStream_t s) {
+void adj_sweep(const AdjTape& T, uint32_t begin, uint32_t end, const double* pk, double* alpha, double* lambda,
+               unsigned long long* delta, hipStream_t s) {
   if (end > begin)
-    hipLaunchKernelGGL(k_adj_sweep, blocks(end - begin), dim3(256), 0, s, T, begin, end, jac, minv, alpha, lambda,
-                       delta);
+    hipLaunchKernelGGL(k_adj_sweep, blocks(end - begin), dim3(256), 0, s, T, begin, end, pk, alpha, lambda, delta);
+}
+bool adj_block(const AdjTape& T, const ColourOffsets& O, uint32_t n, const double* pk, double* alpha, double* lambda,
+               uint32_t sweeps, double tol, unsigned long long* out, hipStream_t s) {
+  if (T.nc <= kAdjHeldContacts && n <= kAdjHeldBodies)
+    hipLaunchKernelGGL((k_adj_block<true, kAdjHeldContacts>), dim3(1), dim3(kAdjHeldContacts), 0, s, T, O, n, pk,
+                       alpha, lambda, sweeps, tol, out);
+  else if (T.nc <= kAdjBlockContacts)
+    hipLaunchKernelGGL((k_adj_block<false, 512>), dim3(1), dim3(512), 0, s, T, O, n, pk, alpha, lambda, sweeps, tol,
+                       out);
+  else return false;
+  return true;
 }
 void adj_assemble(const AdjTape& T, const double* jac, const double* alpha, const double* lambda, double* xbar,
                   double* mubar, hipStream_t s) {
