@@ -82,7 +82,7 @@ static void restore_state(pehip_ctx* ctx, const double* src) {
   hipMemcpyAsync(ctx->w, src + 10 * n, 3 * D * n, hipMemcpyDeviceToDevice, s);
   hipMemcpyAsync(ctx->pnormal, src + 13 * n, 3 * D * n, hipMemcpyDeviceToDevice, s);
   hipMemcpyAsync(ctx->pd, src + 16 * n, D * n, hipMemcpyDeviceToDevice, s);
-  adj_restore_R((uint32_t)n, ctx->q, ctx->R, s);
+  launch_rotations((uint32_t)n, ctx->q, ctx->R, s);
   launch_aabb(ctx->bodies(), s);
 }
 

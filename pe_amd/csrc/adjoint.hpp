@@ -428,7 +428,6 @@ bool adj_block(const AdjTape& T, const struct ColourOffsets& O, uint32_t n, cons
 void adj_assemble(const AdjTape& T, const double* jac, const double* alpha, const double* lambda, double* xbar,
                   double* mubar, hipStream_t s);
 void adj_finish(uint32_t n, const double* alpha, double* vbar, double* wbar, hipStream_t s);
-void adj_restore_R(uint32_t n, const double* q, double* R, hipStream_t s);
 void adj_pack_vel(uint32_t n, const double* v, const double* w, double* vel, hipStream_t s);
 void adj_pack_p(uint32_t nc, const double* f, size_t cap, double* p, double* mu, hipStream_t s);
 

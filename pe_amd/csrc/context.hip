@@ -187,7 +187,7 @@ static void plan_grid(pehip_ctx* ctx, const uint8_t* shape, const double* param,
 // Sphere::update(dq), Union.cpp:306-322, Sphere.cpp:1059); a new position alone translates each
 // member by the union's displacement (Union::setPosition -> Sphere::update(dp), Union.cpp:251-272,
 // Sphere.cpp:1031).  Unions whose pose is unchanged keep their members' positions bit for bit.
-static pehip_status move_members(pehip_ctx* ctx, const double* pos, const double* q, const std::vector<double>& hR) {
+static pehip_status move_members(pehip_ctx* ctx, const double* pos, const double* q) {
   const uint32_t n = ctx->n, nm = ctx->nm;
   const size_t D = sizeof(double);
   std::vector<double> opos(3 * (size_t)n), oq(4 * (size_t)n), mp(3 * (size_t)nm), mr(3 * (size_t)nm);
@@ -204,8 +204,9 @@ static pehip_status move_members(pehip_ctx* ctx, const double* pos, const double
     const bool tra = std::memcmp(&opos[3 * (size_t)i], &pos[3 * (size_t)i], 3 * D) != 0;
     if (!rot && !tra) continue;
     moved = true;
-    m33 R;
-    for (int k = 0; k < 9; ++k) R.a[k] = hR[9 * (size_t)i + k];
+    qd qq;
+    for (int k = 0; k < 4; ++k) qq.v[k] = q[4 * (size_t)i + k];
+    const m33 R = quat_to_R(qq);
     const d3 gp = mk3(pos[3 * (size_t)i], pos[3 * (size_t)i + 1], pos[3 * (size_t)i + 2]);
     const d3 dp = gp - mk3(opos[3 * (size_t)i], opos[3 * (size_t)i + 1], opos[3 * (size_t)i + 2]);
     for (uint32_t m = start[i]; m < start[i + 1]; ++m) {
@@ -537,13 +538,16 @@ pehip_status pehip_upload_members(pehip_ctx* ctx, uint32_t nm, const uint32_t* o
   for (uint32_t i = 0; i < ctx->n; ++i) start[i + 1] += start[i];
   hipSetDevice(ctx->device);
   CK(hipStreamSynchronize(ctx->stream));
-  ctx->free_members();
+  // (the same number of members again: into the arrays that are there)
+  if (nm != ctx->nm || ctx->members_missing) ctx->free_members();
   // a failure below leaves the unions without members: steps refuse to run until an upload succeeds
   const pehip_status st = [&]() -> pehip_status {
     const size_t D = sizeof(double);
-    CK(dalloc(ctx->mstart, (size_t)ctx->n + 1)); CK(dalloc(ctx->mowner, nm)); CK(dalloc(ctx->mmat, nm));
-    CK(dalloc(ctx->msid, nm)); CK(dalloc(ctx->mrad, nm)); CK(dalloc(ctx->mrpos, 3 * (size_t)nm));
-    CK(dalloc(ctx->mpos, 3 * (size_t)nm));
+    if (!ctx->mstart) {
+      CK(dalloc(ctx->mstart, (size_t)ctx->n + 1)); CK(dalloc(ctx->mowner, nm)); CK(dalloc(ctx->mmat, nm));
+      CK(dalloc(ctx->msid, nm)); CK(dalloc(ctx->mrad, nm)); CK(dalloc(ctx->mrpos, 3 * (size_t)nm));
+      CK(dalloc(ctx->mpos, 3 * (size_t)nm));
+    }
     CK(hipMemcpy(ctx->mstart, start.data(), 4 * start.size(), hipMemcpyHostToDevice));
     CK(hipMemcpy(ctx->mowner, owner, 4 * (size_t)nm, hipMemcpyHostToDevice));
     CK(hipMemcpy(ctx->mmat, material, 4 * (size_t)nm, hipMemcpyHostToDevice));
@@ -581,22 +585,17 @@ pehip_status pehip_upload_state(pehip_ctx* ctx, uint32_t n, const double* pos, c
   if (ctx->members_missing) return fail(ctx, PEHIP_INVALID_ARG, "union members not uploaded");
   hipSetDevice(ctx->device);
   CK(hipStreamSynchronize(ctx->stream));
-  std::vector<double> hR(9 * (size_t)n);
-  for (uint32_t i = 0; i < n; ++i) {
-    qd qq;
-    for (int k = 0; k < 4; ++k) qq.v[k] = q[4 * (size_t)i + k];
-    const m33 m = quat_to_R(qq);
-    for (int k = 0; k < 9; ++k) hR[9 * (size_t)i + k] = m.a[k];
-  }
   const size_t D = sizeof(double);
-  if (ctx->nm) CKS(move_members(ctx, pos, q, hR));
+  if (ctx->nm) CKS(move_members(ctx, pos, q));
   CK(hipMemcpy(ctx->pos, pos, 3 * D * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(ctx->q, q, 4 * D * n, hipMemcpyHostToDevice));
-  CK(hipMemcpy(ctx->R, hR.data(), 9 * D * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(ctx->v, v, 3 * D * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(ctx->w, w, 3 * D * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(ctx->pnormal, plane_normal, 3 * D * n, hipMemcpyHostToDevice));
   CK(hipMemcpy(ctx->pd, plane_d, D * n, hipMemcpyHostToDevice));
+  // (the matrices on the device, which evaluates the same expressions: a third of the bytes of an upload
+  // and a pass over the bodies on one host thread less)
+  launch_rotations(n, ctx->q, ctx->R, ctx->stream);
   launch_aabb(ctx->bodies(), ctx->stream);
   return sync_check(ctx);
 }

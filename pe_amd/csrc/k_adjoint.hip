@@ -340,18 +340,6 @@ __global__ void k_adj_finish(uint32_t n, const double* alpha, double* vbar, doub
   }
 }
 
-// Rotation matrices from quaternions and AABBs (restoring a checkpoint on the device).
-__global__ void k_adj_restore_R(uint32_t n, const double* q, double* R) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  qd qq;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) qq.v[k] = q[4 * (size_t)i + k];
-  const m33 m = quat_to_R(qq);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) R[9 * (size_t)i + k] = m.a[k];
-}
-
 // Body-major copy of (v, w) into 6 doubles per body.
 __global__ void k_adj_pack_vel(uint32_t n, const double* v, const double* w, double* vel) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -413,9 +401,6 @@ void adj_assemble(const AdjTape& T, const double* jac, const double* alpha, cons
 }
 void adj_finish(uint32_t n, const double* alpha, double* vbar, double* wbar, hipStream_t s) {
   hipLaunchKernelGGL(k_adj_finish, blocks(n), dim3(256), 0, s, n, alpha, vbar, wbar);
-}
-void adj_restore_R(uint32_t n, const double* q, double* R, hipStream_t s) {
-  hipLaunchKernelGGL(k_adj_restore_R, blocks(n), dim3(256), 0, s, n, q, R);
 }
 void adj_pack_vel(uint32_t n, const double* v, const double* w, double* vel, hipStream_t s) {
   hipLaunchKernelGGL(k_adj_pack_vel, blocks(n), dim3(256), 0, s, n, v, w, vel);

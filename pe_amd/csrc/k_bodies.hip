@@ -10,6 +10,15 @@ __global__ void k_aabb(Bodies B) {
   if (i < B.n) update_aabb(B, i);
 }
 
+// Rotation matrices from the quaternions (Quaternion::toRotationMatrix), as the host computes them.
+__global__ void k_rotations(uint32_t n, const double* q, double* R) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const m33 m = quat_to_R(ld4(q, i));
+#pragma unroll
+  for (int k = 0; k < 9; ++k) R[9 * (size_t)i + k] = m.a[k];
+}
+
 // Body caching (predicted velocities, solver body records); see predict_body.
 __global__ void k_predict(Bodies B, d3 gravity, double dt) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -46,6 +55,9 @@ __global__ void k_kinetic(Bodies B, double* partial) {
 
 void launch_aabb(const Bodies& B, hipStream_t s) {
   if (B.n) hipLaunchKernelGGL(k_aabb, dim3((B.n + 255) / 256), dim3(256), 0, s, B);
+}
+void launch_rotations(uint32_t n, const double* q, double* R, hipStream_t s) {
+  if (n) hipLaunchKernelGGL(k_rotations, dim3((n + 255) / 256), dim3(256), 0, s, n, q, R);
 }
 void launch_predict(const Bodies& B, d3 g, double dt, hipStream_t s) {
   if (B.n) hipLaunchKernelGGL(k_predict, dim3((B.n + 255) / 256), dim3(256), 0, s, B, g, dt);

@@ -83,6 +83,7 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32
                       size_t n, int bits, uint32_t* scratch, hipStream_t s);
 
 void launch_aabb(const Bodies& B, hipStream_t s);
+void launch_rotations(uint32_t n, const double* q, double* R, hipStream_t s);
 void launch_predict(const Bodies& B, d3 g, double dt, hipStream_t s);
 void launch_integrate(const Bodies& B, double dt, double damping, bool exact_trig, hipStream_t s);
 void launch_eval_trig(int fn, bool exact, size_t n, const double* x, const double* y, double* out, hipStream_t s);

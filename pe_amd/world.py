@@ -147,6 +147,8 @@ class World:
         self._bodies_dirty = True
         self._params_dirty = True
         self._state_on_device = False
+        self._state_set = False  # the device's state is one that setState gave, not a step's
+        self._m_static = None    # member arrays for the upload, as long as the members stay the same
         self.timestep = 0
 
     # ------------------------------------------------------------------ settings
@@ -265,12 +267,14 @@ class World:
     # ------------------------------------------------------------------ bodies
     def _sync_from_device(self):
         if self._state_on_device and self._ctx is not None:
-            st = self.getState()
+            # (not getState, which would first upload changed bodies over the state to be read)
+            st = self._read_state()
             mg = st.pop("mgpos", None)
             self._arrays.update(st)
             if mg is not None:
                 self._m_gpos = list(mg)
             self._state_on_device = False
+            self._state_set = False
 
     def _materialise_lists(self):
         if self._arrays is not None:
@@ -404,6 +408,7 @@ class World:
         idx = self._add(UNION, spheres[0][2], False, union_param(rpos, [r for _, r, _ in spheres]), g,
                         (1.0, 0.0, 0.0, 0.0), inv_mass, np.asarray(I), Iinv, (0.0, 0.0, 0.0), 0.0, uid)
         self._u_mass[idx] = mass
+        self._m_static = None
         for k in range(n):
             self._m_owner.append(idx)
             self._m_sid.append(self._next_sid)
@@ -474,6 +479,7 @@ class World:
             lst[body] = lst[last]
             lst.pop()
         if self._m_owner:
+            self._m_static = None
             # the removed union's members leave; the moved body's follow it; members stay grouped
             # by union in body order, each union's in its own order (a stable sort)
             owner = [body if o == last else o for o in self._m_owner]
@@ -535,6 +541,7 @@ class World:
             for u in unions:
                 sel = np.flatnonzero(owner == u)
                 arrays["param"][u] = union_param(rpos[sel], rad[sel])
+            self._m_static = None
             self._m_owner = owner.tolist()
             self._m_sid = [int(x) for x in members["sid"]]
             self._m_uid = [int(x) for x in members.get("uid", np.asarray(arrays["uid"])[owner])]
@@ -624,20 +631,23 @@ class World:
             self._bodies_dirty = False
             self._state_on_device = False
 
-    def _upload_members(self):
-        """Union members to the device (after their union bodies)."""
+    def _upload_members(self, gpos=None):
+        """Union members to the device (after their union bodies), at gpos or where they are."""
         k = len(self._m_owner)
-        mo = np.ascontiguousarray(self._m_owner, np.uint32)
-        ms = np.ascontiguousarray(self._m_sid, np.uint64)
-        mm = np.ascontiguousarray(self._m_mat, np.uint32)
-        mr = np.ascontiguousarray(self._m_rad, float)
-        mrp = np.ascontiguousarray(np.asarray(self._m_rpos, float).reshape(k, 3))
-        mg = np.ascontiguousarray(np.asarray(self._m_gpos, float).reshape(k, 3))
+        if self._m_static is None:
+            self._m_static = (np.ascontiguousarray(self._m_owner, np.uint32),
+                              np.ascontiguousarray(self._m_sid, np.uint64),
+                              np.ascontiguousarray(self._m_mat, np.uint32), np.ascontiguousarray(self._m_rad, float),
+                              np.ascontiguousarray(np.asarray(self._m_rpos, float).reshape(k, 3)))
+        mo, ms, mm, mr, mrp = self._m_static
+        mg = np.ascontiguousarray(np.asarray(self._m_gpos if gpos is None else gpos, float).reshape(k, 3))
         check(_abi.load().pehip_upload_members(self._ctx, k, ptr(mo, _abi._U32), ptr(ms, _abi._U64),
                                                ptr(mm, _abi._U32), ptr(mr), ptr(mrp), ptr(mg)), self._ctx)
 
     def close(self):
         if self._ctx is not None:
+            if self._state_set:       # the state given last stays the world's
+                self._sync_from_device()
             _abi.load().pehip_destroy(self._ctx)
             self._ctx = None
 
@@ -662,6 +672,7 @@ class World:
         self._ensure_device()
         check(_abi.load().pehip_step(self._ctx, float(dt), int(steps)), self._ctx)
         self._state_on_device = True
+        self._state_set = False
         self.timestep += int(steps)
 
     def detect(self):
@@ -687,6 +698,9 @@ class World:
     # ------------------------------------------------------------------ state
     def getState(self):
         self._ensure_device()
+        return self._read_state()
+
+    def _read_state(self):
         n = self.size
         st = {"pos": np.zeros((n, 3)), "q": np.zeros((n, 4)), "v": np.zeros((n, 3)), "w": np.zeros((n, 3)),
               "normal": np.zeros((n, 3)), "d": np.zeros(n)}
@@ -706,13 +720,12 @@ class World:
         self._ensure_device()
         check(_abi.load().pehip_upload_state(self._ctx, n, ptr(c["pos"]), ptr(c["q"]), ptr(c["v"]), ptr(c["w"]),
                                              ptr(c["normal"]), ptr(c["d"])), self._ctx)
-        if self._arrays is not None:
-            for k in c:
-                self._arrays[k] = c[k].copy()
         if "mgpos" in st and self._m_owner:   # union members are placed as given
-            self._m_gpos = list(np.asarray(st["mgpos"], float).reshape(-1, 3))
-            self._upload_members()
-        self._state_on_device = False
+            self._upload_members(st["mgpos"])
+            if self._arrays is None:
+                self._m_gpos = list(np.array(st["mgpos"], float).reshape(-1, 3))
+        # the host arrays follow when they are asked for
+        self._state_on_device = self._state_set = self._arrays is not None
 
     def contacts(self):
         L = _abi.load()
