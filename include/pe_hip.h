@@ -79,9 +79,9 @@ typedef struct {
 } pehip_params;
 
 typedef enum {
-  /* one workgroup for few contacts (models with a search, 3 and 5: up to 16; the others: up to 768);
-   * beyond them, abort_threshold <= 0: dataflow when the step's contacts fit it (65,536), else colour
-   * launches; abort_threshold > 0: colour launches */
+  /* one workgroup for up to 768 contacts of the models without a search (all but 3 and 5); otherwise
+   * abort_threshold <= 0: dataflow when the step's contacts fit it (65,536), else colour launches;
+   * abort_threshold > 0: colour launches */
   PEHIP_SCHEDULE_AUTO = 0,
   /* one kernel launch per colour and sweep */
   PEHIP_SCHEDULE_COLOUR_LAUNCHES = 1,

@@ -413,7 +413,7 @@ __device__ bool scene_step(const Bodies& B, const RawContacts& R, const SolverCo
       for (int it = 0; it < A.iters; ++it) {
         double dmax = 0;
         for (uint32_t k = 0; k < ncol; ++k) {
-          dmax = smax(dmax, resident_relax<MODEL, Trig, true>(r, colour == k, ldvw, A.max_sub));
+          if (colour == k) dmax = smax(dmax, resident_relax<MODEL, Trig>(r, ldvw, A.max_sub));
           __syncthreads();
         }
         iters = it + 1;

@@ -27,20 +27,18 @@ constexpr uint32_t kDataflowSpinLimit = 1u << 22;
 // With an abort threshold the host reads the device's stop flag once per this many sweeps.
 constexpr uint32_t kAbortPoll = 32;
 // Automatic schedule: one workgroup runs all sweeps of a step while it holds all the contacts on the chip
-// (models without a search), or up to a few contacts (models with one).  A colour costs it 1 to 2 us; an
-// update costs the dataflow sweeps about 4 us, and so does a colour launch, the choice with an abort
-// threshold.  But it relaxes only four sliding contacts at a time.  50 sweeps, one workgroup against
-// dataflow: model 1 0.22 against 0.41 ms (18 contacts), 0.22 against 0.65 (100), 0.23 against 0.63 (194), 0.43
-// against 0.66 (281), 0.48 against 0.70 (408); model 3 0.17 against 0.27 (5), 0.44 against 0.50 (18), 0.96
-// against 0.79 (39), 3.2 against 1.0 (144).
-constexpr uint32_t kSingleBlockMaxContacts = kResidentWide, kSingleBlockMaxSearching = 16;
+// (models without a search).  A colour costs it 1 to 2 us; an update costs the dataflow sweeps about 4 us, and
+// so does a colour launch, the choice with an abort threshold.  50 sweeps of model 1, one workgroup against
+// dataflow: 0.22 against 0.41 ms (18 contacts), 0.22 against 0.65 (100), 0.23 against 0.63 (194), 0.43 against
+// 0.66 (281), 0.48 against 0.70 (408).  (Models with a search: a workgroup relaxes four sliding contacts at a
+// time; model 3 0.44 against 0.50 (18), 0.96 against 0.79 (39), 3.2 against 1.0 (144).)
+constexpr uint32_t kSingleBlockMaxContacts = kResidentWide;
 
-bool is_searching(int model) { return model == PEHIP_INELASTIC_COULOMB_DECOUPLING || model == PEHIP_INELASTIC_GMD; }
-
-// The automatic schedule's choice of one workgroup for a step of nc contacts.
 bool choose_single_block(const pehip_params& P, uint32_t nc) {
-  return nc <= (is_searching(P.relaxation_model) ? kSingleBlockMaxSearching : kSingleBlockMaxContacts);
+  return P.relaxation_model != PEHIP_INELASTIC_COULOMB_DECOUPLING && P.relaxation_model != PEHIP_INELASTIC_GMD &&
+         nc <= kSingleBlockMaxContacts;
 }
+
 std::string g_create_error;
 
 uint32_t next_pow2(uint64_t x) {

@@ -203,10 +203,9 @@ __global__ void __launch_bounds__(THREADS) k_sweep_resident(SolverContacts C, Co
   const uint32_t nc = O.off[O.ncol];
   for (uint32_t i = tid; i < kTable; i += THREADS) body[i] = kNoBody;
   __syncthreads();
-  // With a search a colour's slots, which follow one another, are spread over the wavefronts, which relax
-  // their sliding contacts one by one; without, they stay together, so that the other wavefronts pass a
-  // colour by (72 contacts of a colour in all of 12 wavefronts: 7 us a colour).
-  const uint32_t slot = MODEL == 3 || MODEL == 5 ? lane * (THREADS / 64) + wave : tid;
+  // a colour's slots, which follow one another, stay together, so that the other wavefronts pass the colour
+  // by (72 contacts of a colour spread over all of 12 wavefronts: 7 us a colour instead of 2.3)
+  const uint32_t slot = tid;
   const bool have = slot < nc;
   uint32_t colour = kMaxColours;
   auto place = [&](uint32_t b) {
@@ -232,9 +231,7 @@ __global__ void __launch_bounds__(THREADS) k_sweep_resident(SolverContacts C, Co
     // non-negative doubles (and NaN above +inf) order like their bit patterns
     unsigned long long u = 0;
     for (uint32_t k = 0; k < O.ncol; ++k) {
-      const unsigned long long d =
-          (unsigned long long)__double_as_longlong(resident_relax<MODEL, Trig, kHold>(r, colour == k, ldvw, maxSub));
-      u = d > u ? d : u;
+      if (colour == k) u = (unsigned long long)__double_as_longlong(resident_relax<MODEL, Trig>(r, ldvw, maxSub));
       __syncthreads();
     }
     ++it;
@@ -275,9 +272,7 @@ static void resident_dispatch(int model, const SolverContacts& C, const ColourOf
     case 0: if (wide) PE_RESIDENT(0, kResidentWide); else PE_RESIDENT(0, kResidentThreads); break;
     case 1: if (wide) PE_RESIDENT(1, kResidentWide); else PE_RESIDENT(1, kResidentThreads); break;
     case 2: if (wide) PE_RESIDENT(2, kResidentWide); else PE_RESIDENT(2, kResidentThreads); break;
-    case 4: if (wide) PE_RESIDENT(4, kResidentWide); else PE_RESIDENT(4, kResidentThreads); break;
-    case 5: PE_RESIDENT(5, kResidentThreads); break;
-    default: PE_RESIDENT(3, kResidentThreads); break;
+    default: if (wide) PE_RESIDENT(4, kResidentWide); else PE_RESIDENT(4, kResidentThreads); break;
   }
 #undef PE_RESIDENT
 }
@@ -347,8 +342,7 @@ static void block_dispatch(int model, const SolverContacts& C, const ColourOffse
 void launch_sweep_block(int model, bool exact_trig, const SolverContacts& C, const ColourOffsets& O, uint32_t iters,
                         const Bodies& B, double dtinv, int maxSub, double thr, unsigned long long* deltas,
                         hipStream_t s) {
-  const bool searches = model == 3 || model == 5;
-  if (O.off[O.ncol] <= (searches ? kResidentThreads : kResidentWide)) {
+  if (model != 3 && model != 5 && O.off[O.ncol] <= kResidentWide) {
     if (exact_trig) resident_dispatch<TrigExact>(model, C, O, iters, B, maxSub, thr, deltas, s);
     else resident_dispatch<TrigFast>(model, C, O, iters, B, maxSub, thr, deltas, s);
     return;
