@@ -646,10 +646,12 @@ class World:
 
     def close(self):
         if self._ctx is not None:
-            if self._state_set:       # the state given last stays the world's
-                self._sync_from_device()
-            _abi.load().pehip_destroy(self._ctx)
-            self._ctx = None
+            try:
+                if self._state_set:       # the state given last stays the world's
+                    self._sync_from_device()
+            finally:                      # also where the device no longer answers
+                ctx, self._ctx = self._ctx, None
+                _abi.load().pehip_destroy(ctx)
 
     def __del__(self):
         try:

@@ -1,0 +1,111 @@
+"""The world's host state without a device: the C library is a stand-in that keeps the arrays it is given."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from pe_amd import World, _abi
+from pe_amd._abi import PeHipError
+
+FIELDS = (("pos", 3), ("q", 4), ("v", 3), ("w", 3), ("normal", 3), ("d", 1))
+
+
+class Library:
+    """Bodies of one context.  A step moves every body and member by one in x and fails where told to."""
+
+    def __init__(self):
+        self.state, self.members, self.alive, self.fail = {}, None, 0, ()
+
+    def __getattr__(self, name):
+        if not name.startswith("pehip_"):
+            raise AttributeError(name)
+        return lambda *a: 3 if name in self.fail else (getattr(self, "do_" + name[6:], lambda *b: 0)(*a) or 0)
+
+    def pehip_last_error(self, ctx):
+        return b"refused"
+
+    def do_create(self, params, device, out):
+        ctypes.cast(out, ctypes.POINTER(ctypes.c_void_p))[0] = 1
+        self.alive += 1
+
+    def do_destroy(self, ctx):
+        self.alive -= 1
+
+    def take(self, n, arrays):
+        for (k, w), p in zip(FIELDS, arrays):
+            self.state[k] = np.ctypeslib.as_array(p, (n, w)).copy()
+
+    def do_upload_bodies(self, ctx, n, shape, sid, mat, fixed, param, pos, q, v, w, im, inertia, inverse, normal, d):
+        self.take(n, (pos, q, v, w, normal, d))
+
+    def do_upload_state(self, ctx, n, *arrays):
+        before = self.state["pos"]
+        self.take(n, arrays)
+        if self.members is not None:                  # one union, the last body
+            self.members = self.members + (self.state["pos"] - before)[-1]
+
+    def do_download_state(self, ctx, n, *arrays):
+        for (k, w), p in zip(FIELDS, arrays):
+            np.ctypeslib.as_array(p, (n, w))[:] = self.state[k]
+
+    def do_upload_members(self, ctx, k, owner, sid, mat, rad, rpos, gpos):
+        given = np.ctypeslib.as_array(gpos, (k, 3))
+        if not np.isfinite(given).all():
+            return 1
+        self.members = given.copy()
+
+    def do_download_members(self, ctx, k, gpos):
+        np.ctypeslib.as_array(gpos, (k, 3))[:] = self.members
+
+    def do_step(self, ctx, dt, steps):
+        for _ in range(steps):
+            self.state["pos"][:, 0] += 1.0
+            if self.members is not None:
+                self.members[:, 0] += 1.0
+        return 3 if "step" in self.fail else 0
+
+
+@pytest.fixture
+def lib(monkeypatch):
+    library = Library()
+    monkeypatch.setattr(_abi, "load", lambda: library)
+    # the pointers stand for arrays of doubles
+    monkeypatch.setattr("pe_amd.world.ptr", lambda a, typ=None: None if a is None else a.ctypes.data_as(
+        ctypes.POINTER(np.ctypeslib.as_ctypes_type(a.dtype))))
+    return library
+
+
+def world(union=False):
+    w = World()
+    m = w.createMaterial("m", 1000.0, 0.0, 0.1, 0.1)
+    w.createPlane(0, (0.0, 0.0, 1.0), 0.0, m)
+    for k in range(3):
+        w.createSphere(k + 1, (2.0 * k, 0.0, 1.0), 0.5, m)
+    if union:
+        w.createUnion(9, (0.0, 5.0, 1.0), [((0.0, 0.0, 0.0), 0.3, m), ((0.4, 0.0, 0.0), 0.3, m)])
+    return w
+
+
+def another(w, by):
+    """Another state of the world, and a copy that no call has seen."""
+    st = {k: v + by for k, v in w.getState().items()}
+    return st, {k: v.copy() for k, v in st.items()}
+
+
+def equal(a, b):
+    for k, n in FIELDS:
+        assert np.array_equal(np.reshape(a[k], (-1, n)), np.reshape(b[k], (-1, n))), k
+
+
+def test_close_frees_the_context_whatever_fails(lib):
+    w = world()
+    st, _ = another(w, 0.25)
+    w.setState(st)
+    lib.fail = ("pehip_download_state", "pehip_download_members")
+    try:
+        w.close()
+    except PeHipError:
+        pass
+    assert lib.alive == 0 and w._ctx is None
+    w.close()
+    assert lib.alive == 0
