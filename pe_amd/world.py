@@ -147,7 +147,6 @@ class World:
         self._bodies_dirty = True
         self._params_dirty = True
         self._state_on_device = False
-        self._state_set = False  # the device's state is one that setState gave, not a step's
         self._m_static = None    # member arrays for the upload, as long as the members stay the same
         self.timestep = 0
 
@@ -272,9 +271,8 @@ class World:
             mg = st.pop("mgpos", None)
             self._arrays.update(st)
             if mg is not None:
-                self._m_gpos = list(mg)
+                self._m_gpos = mg
             self._state_on_device = False
-            self._state_set = False
 
     def _materialise_lists(self):
         if self._arrays is not None:
@@ -409,6 +407,7 @@ class World:
                         (1.0, 0.0, 0.0, 0.0), inv_mass, np.asarray(I), Iinv, (0.0, 0.0, 0.0), 0.0, uid)
         self._u_mass[idx] = mass
         self._m_static = None
+        self._m_gpos = list(self._m_gpos)     # (rows of an array where a state was set or read back)
         for k in range(n):
             self._m_owner.append(idx)
             self._m_sid.append(self._next_sid)
@@ -433,7 +432,7 @@ class World:
         return {"owner": np.asarray(self._m_owner, np.uint32), "sid": np.asarray(self._m_sid, np.uint64),
                 "uid": np.asarray(self._m_uid, np.uint64),
                 "mat": np.asarray(self._m_mat, np.uint32), "radius": np.asarray(self._m_rad, float),
-                "rpos": np.asarray(self._m_rpos, float).reshape(k, 3), "gpos": np.asarray(self._m_gpos, float).reshape(k, 3)}
+                "rpos": np.asarray(self._m_rpos, float).reshape(k, 3), "gpos": np.array(self._m_gpos, float).reshape(k, 3)}
 
     def createPlane(self, uid, normal, d, material):
         """createPlane (Plane.cpp:1202-1240) and the Plane ctor (Plane.cpp:77-102)."""
@@ -631,8 +630,8 @@ class World:
             self._bodies_dirty = False
             self._state_on_device = False
 
-    def _upload_members(self, gpos=None):
-        """Union members to the device (after their union bodies), at gpos or where they are."""
+    def _upload_members(self):
+        """Union members to the device (after their union bodies)."""
         k = len(self._m_owner)
         if self._m_static is None:
             self._m_static = (np.ascontiguousarray(self._m_owner, np.uint32),
@@ -640,18 +639,14 @@ class World:
                               np.ascontiguousarray(self._m_mat, np.uint32), np.ascontiguousarray(self._m_rad, float),
                               np.ascontiguousarray(np.asarray(self._m_rpos, float).reshape(k, 3)))
         mo, ms, mm, mr, mrp = self._m_static
-        mg = np.ascontiguousarray(np.asarray(self._m_gpos if gpos is None else gpos, float).reshape(k, 3))
+        mg = np.ascontiguousarray(np.asarray(self._m_gpos, float).reshape(k, 3))
         check(_abi.load().pehip_upload_members(self._ctx, k, ptr(mo, _abi._U32), ptr(ms, _abi._U64),
                                                ptr(mm, _abi._U32), ptr(mr), ptr(mrp), ptr(mg)), self._ctx)
 
     def close(self):
         if self._ctx is not None:
-            try:
-                if self._state_set:       # the state given last stays the world's
-                    self._sync_from_device()
-            finally:                      # also where the device no longer answers
-                ctx, self._ctx = self._ctx, None
-                _abi.load().pehip_destroy(ctx)
+            _abi.load().pehip_destroy(self._ctx)
+            self._ctx = None
 
     def __del__(self):
         try:
@@ -674,7 +669,6 @@ class World:
         self._ensure_device()
         check(_abi.load().pehip_step(self._ctx, float(dt), int(steps)), self._ctx)
         self._state_on_device = True
-        self._state_set = False
         self.timestep += int(steps)
 
     def detect(self):
@@ -709,9 +703,13 @@ class World:
         check(_abi.load().pehip_download_state(self._ctx, n, ptr(st["pos"]), ptr(st["q"]), ptr(st["v"]),
                                                ptr(st["w"]), ptr(st["normal"]), ptr(st["d"])), self._ctx)
         if self._m_owner:   # union members' global positions
-            st["mgpos"] = np.zeros((len(self._m_owner), 3))
-            check(_abi.load().pehip_download_members(self._ctx, len(self._m_owner), ptr(st["mgpos"])), self._ctx)
+            st["mgpos"] = self._read_members()
         return st
+
+    def _read_members(self):
+        mg = np.zeros((len(self._m_owner), 3))
+        check(_abi.load().pehip_download_members(self._ctx, len(self._m_owner), ptr(mg)), self._ctx)
+        return mg
 
     def setState(self, st):
         n = self.size
@@ -722,12 +720,18 @@ class World:
         self._ensure_device()
         check(_abi.load().pehip_upload_state(self._ctx, n, ptr(c["pos"]), ptr(c["q"]), ptr(c["v"]), ptr(c["w"]),
                                              ptr(c["normal"]), ptr(c["d"])), self._ctx)
-        if "mgpos" in st and self._m_owner:   # union members are placed as given
-            self._upload_members(st["mgpos"])
-            if self._arrays is None:
-                self._m_gpos = list(np.array(st["mgpos"], float).reshape(-1, 3))
-        # the host arrays follow when they are asked for
-        self._state_on_device = self._state_set = self._arrays is not None
+        # the host's state is the one given, whatever becomes of the steps that follow, of the context, of
+        # the arrays given or of those handed out before
+        if self._arrays is not None:
+            for k in c:
+                self._arrays[k] = c[k].copy()
+        self._state_on_device = False
+        if self._m_owner:
+            if "mgpos" in st:                 # union members are placed as given
+                self._m_gpos = np.array(st["mgpos"], float).reshape(-1, 3)
+                self._upload_members()
+            else:                             # or where their unions took them
+                self._m_gpos = self._read_members()
 
     def contacts(self):
         L = _abi.load()

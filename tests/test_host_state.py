@@ -14,7 +14,7 @@ class Library:
     """Bodies of one context.  A step moves every body and member by one in x and fails where told to."""
 
     def __init__(self):
-        self.state, self.members, self.alive, self.fail = {}, None, 0, ()
+        self.state, self.members, self.alive, self.fail, self.worlds = {}, None, 0, (), []
 
     def __getattr__(self, name):
         if not name.startswith("pehip_"):
@@ -72,11 +72,14 @@ def lib(monkeypatch):
     # the pointers stand for arrays of doubles
     monkeypatch.setattr("pe_amd.world.ptr", lambda a, typ=None: None if a is None else a.ctypes.data_as(
         ctypes.POINTER(np.ctypeslib.as_ctypes_type(a.dtype))))
-    return library
+    yield library
+    for w in library.worlds:
+        w._ctx = None                  # no handle of the stand-in's reaches the real library
 
 
-def world(union=False):
+def world(lib, union=False):
     w = World()
+    lib.worlds.append(w)
     m = w.createMaterial("m", 1000.0, 0.0, 0.1, 0.1)
     w.createPlane(0, (0.0, 0.0, 1.0), 0.0, m)
     for k in range(3):
@@ -98,7 +101,7 @@ def equal(a, b):
 
 
 def test_close_frees_the_context_whatever_fails(lib):
-    w = world()
+    w = world(lib)
     st, _ = another(w, 0.25)
     w.setState(st)
     lib.fail = ("pehip_download_state", "pehip_download_members")
@@ -109,3 +112,76 @@ def test_close_frees_the_context_whatever_fails(lib):
     assert lib.alive == 0 and w._ctx is None
     w.close()
     assert lib.alive == 0
+
+
+def test_the_state_given_outlives_steps_and_the_context(lib):
+    w = world(lib)
+    st, given = another(w, 0.25)
+    w.setState(st)
+    for v in st.values():
+        v += 1.0                       # the caller's arrays are the caller's
+    w.run(3, 1e-3)
+    w.close()                          # the steps' state was never asked for
+    equal(w.host_arrays(), given)
+    i = w.createSphere(9, (9.0, 9.0, 9.0), 0.5, 0)
+    now = w.getState()                 # a new context, from the host's state
+    equal({k: v[:i] for k, v in now.items()}, given)
+
+
+def test_the_state_given_is_kept_where_a_run_fails_part_way(lib):
+    w = world(lib)
+    st, given = another(w, 0.25)
+    w.setState(st)
+    lib.fail = ("pehip_step",)
+    lib.do_step(None, 0.0, 2)          # two steps were done
+    with pytest.raises(PeHipError):
+        w.run(4, 1e-3)
+    equal(w.host_arrays(), given)
+
+
+def test_a_held_dict_follows_and_keeps_what_is_written_into_it(lib):
+    w = world(lib)
+    held = w.host_arrays()
+    before = held["pos"]
+    kept = before.copy()
+    st, given = another(w, 0.25)
+    w.setState(st)
+    equal(held, given)
+    assert np.array_equal(before, kept)            # the array of before is not written over
+    held["v"][1] = (1.0, 2.0, 3.0)
+    given["v"][1] = (1.0, 2.0, 3.0)
+    equal(w.host_arrays(), given)
+
+
+def test_members_on_the_host_follow_the_state_given(lib):
+    w = world(lib, union=True)
+    st, given = another(w, 0.25)
+    w.setState(st)
+    st["mgpos"] += 1.0
+    w.members()["gpos"][:] = 0.0
+    assert np.array_equal(w.members()["gpos"], given["mgpos"])
+    w.run(2, 1e-3)
+    w.close()
+    equal(w.host_arrays(), given)
+    assert np.array_equal(w.members()["gpos"], given["mgpos"])
+    w = world(lib, union=True)
+    st, given = another(w, 0.25)
+    del st["mgpos"]                                # the unions take their members along
+    w.setState(st)
+    assert np.array_equal(w.members()["gpos"], given["mgpos"])
+    w.createMaterial("other", 1000.0, 0.0, 0.1, 0.1)
+    assert np.array_equal(w.getState()["mgpos"], given["mgpos"])
+    w.createUnion(10, (0.0, 9.0, 1.0), [((0.0, 0.0, 0.0), 0.3, 0)])
+    assert np.array_equal(w.members()["gpos"][:2], given["mgpos"])
+
+
+def test_the_state_given_is_the_hosts_where_its_members_are_refused(lib):
+    w = world(lib, union=True)
+    st, given = another(w, 0.25)
+    st["mgpos"][1, 2] = np.nan
+    with pytest.raises(PeHipError):
+        w.setState(st)
+    equal(w.host_arrays(), given)
+    equal(w.getState(), given)
+    w.setState(given)                              # and a good one is taken again
+    assert np.array_equal(w.members()["gpos"], given["mgpos"])
