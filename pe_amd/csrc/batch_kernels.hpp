@@ -363,17 +363,19 @@ __device__ bool scene_step(const Bodies& B, const RawContacts& R, const SolverCo
   }
 
   // ---- sweeps.  Scenes of at most T contacts of a model without a search: everything on the chip, see
-  // resident.hpp.  The models with a search (3 and 5), by at most 256 threads, in two parts a colour: every
-  // contact by one lane, except that the sliding ones go on a list (in tab: a colour's contacts share no
+  // resident.hpp.  Model 3, by at most 256 threads, in two parts a colour: every contact by one lane, except that the sliding ones go on a list (in tab: a colour's contacts share no
   // non-fixed body, so it holds them), which the wavefronts then take one contact at a time.  A colour of a
   // scene holds few contacts, of which up to a third slide; a lane's search takes 12.6k cycles a pass however
-  // few of its wavefront's lanes search, a wavefront's 3.0k to 3.7k.  (Measured for these models too: the
+  // few of its wavefront's lanes search, a wavefront's 3.0k to 3.7k.  (Measured for this model too: the
   // contacts on the chip, each wavefront relaxing its own sliding ones: 100 against 89 ms for ten steps of
   // 640 scenes of 50 to 2,000 spheres, because the sliding contacts of a colour, five on average, fall
   // unevenly on the wavefronts.)  Ten steps of 1,500 scenes of 40 to 100 spheres: 37 ms with one lane a
   // contact, 27 now; of 640 scenes of 50 to 2,000: 135 and 96.
-  constexpr bool kSearch = MODEL == 3 || MODEL == 5;
-  constexpr bool kSearches = kSearch && MAXT <= 256, kResident = !kSearch && MAXT <= kResidentThreads;
+  // Model 5 stays with one lane a contact and the 512-thread kernel: its tree search takes a wavefront so long that
+  // lists made its batches up to 2.2 times slower (10 steps of 1,500 settled scenes of 200 to 600 spheres: 239 ms
+  // by lanes, 527 with lists; of 640 scenes of 50 to 2,000, still falling: 59 and 86).
+  constexpr bool kSearches = MODEL == 3 && MAXT <= 256;
+  constexpr bool kResident = MODEL != 3 && MODEL != 5 && MAXT <= kResidentThreads;
   // Three counts in turn: the one of the colour before is cleared between this colour's first barrier,
   // when every thread has read it, and the next colour's, behind which it is used again.
   uint32_t* slide_count = red + 13;    // (the scans use the first eight words)
@@ -539,7 +541,7 @@ static void batch_dispatch(int model, const Bodies& B, const RawContacts& R, con
 template <class Trig>
 static void batch_dispatch_threads(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C,
                                    const BatchArgs& A, uint32_t grid, uint32_t threads, hipStream_t s) {
-  if (threads <= 256) batch_dispatch<Trig, 256>(model, B, R, C, A, grid, threads, s);
+  if (threads <= 256 && model != 5) batch_dispatch<Trig, 256>(model, B, R, C, A, grid, threads, s);
   else batch_dispatch<Trig, kBatchMaxThreads>(model, B, R, C, A, grid, threads, s);
 }
 
