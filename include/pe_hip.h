@@ -334,7 +334,9 @@ typedef struct pehip_batch pehip_batch;
 /* Launch configuration of the batched step (chosen by pehip_batch_autotune or set by hand). */
 typedef struct {
   uint32_t threads;          /* workgroup size per scene: 64, 128, 256 or 512 */
-  uint32_t blocks_per_cu;    /* persistent workgroups per compute unit (1..16) */
+  uint32_t blocks_per_cu;    /* persistent workgroups per compute unit (1..16); a unit runs 512 threads at a time,
+                              * 256 where few or small scenes let a wavefront take a SIMD's whole register file, and
+                              * the others queue */
   uint32_t steps_per_launch; /* time steps a workgroup advances a scene before taking the next */
   uint32_t use_graph;        /* 1: replay the launches of pehip_batch_step from a captured hipGraph */
 } pehip_batch_tuning;

@@ -54,6 +54,7 @@ struct pehip_batch {
 
   // scenes
   uint32_t nscenes = 0;
+  uint32_t largest = 0;  // bodies of the largest scene
   std::vector<SceneInfo> hinfo;
   std::vector<uint32_t> hplane_idx;
   SceneInfo* info = nullptr;
@@ -189,10 +190,30 @@ static uint32_t grid_of(const pehip_batch* b, const pehip_batch_tuning& t) {
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(g, b->nscenes));
 }
 
+// The wide kernel (see k_batch) halves the workgroups in flight.  It is taken where that costs nothing -- they
+// all fit at one wavefront a SIMD, or the largest scene takes longer than its share of the CUs' work takes them --
+// and with model 3 also for scenes of up to 100 bodies on average, whose sliding contacts it relaxes three times as
+// fast.  Model 5 gains nothing from it.  10 steps (piles), 3 steps (lattices) with 256 threads, the narrow kernel
+// against the wide one:
+//   model 3  200 scenes of 50 to 2,000 spheres    546 and 369 ms    640 of them   577 and 396
+//            1,500 settled scenes of 40 to 100    105 and 74        of 200 to 600  669 and 820
+//            1,024 lattices of 90 to 400           82 and 96
+//            5 steps of 1,100 settled scenes of 50 to 90 bodies: 47 and 30; 80 to 130: 99 and 94; 110 to 170: 136 and 145
+//            (lattices of 60 to 80 bodies, which fall apart in a few steps: 81 and 85)
+//   model 1  640 scenes of 50 to 2,000            20 and 16        1,024 lattices of 300 to 2,000   68 and 80
+//            1,500 scenes of 40 to 100            6.4 and 9.8       1,500 settled of 200 to 600     78 and 112
+static bool batch_wide(const pehip_batch* b, const pehip_batch_tuning& t) {
+  const int model = b->prm.relaxation_model;
+  if (t.threads > kBatchWideThreads || model == PEHIP_INELASTIC_GMD) return false;
+  const uint64_t slots = (uint64_t)b->ncu * (kBatchWideThreads / t.threads);
+  if (grid_of(b, t) <= slots || b->n <= slots * b->largest) return true;
+  return model == PEHIP_INELASTIC_COULOMB_DECOUPLING && b->n <= 100ull * b->nscenes;
+}
+
 static void enqueue_launch(pehip_batch* b, const BatchArgs& A, uint32_t add_steps) {
   launch_batch_begin(b->queue, add_steps, b->stream);
   launch_batch(b->prm.relaxation_model, b->prm.exact_trig != 0, b->bodies(), b->raw, b->sol, A, grid_of(b, b->tun),
-               b->tun.threads, b->stream);
+               b->tun.threads, batch_wide(b, b->tun), b->stream);
   b->launches += 2;
 }
 
@@ -205,7 +226,7 @@ static pehip_status capture_graph(pehip_batch* b, double dt) {
   BK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   launch_batch_begin(b->queue, b->tun.steps_per_launch, b->stream);
   launch_batch(b->prm.relaxation_model, b->prm.exact_trig != 0, b->bodies(), b->raw, b->sol, A, grid_of(b, b->tun),
-               b->tun.threads, b->stream);
+               b->tun.threads, batch_wide(b, b->tun), b->stream);
   BK(hipStreamEndCapture(b->stream, &g));
   const hipError_t e = hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0);
   hipGraphDestroy(g);
@@ -445,6 +466,8 @@ pehip_status pehip_batch_upload(pehip_batch* b, uint32_t nscenes, const uint32_t
   const pehip_status st = [&]() -> pehip_status {
     b->n = n;
     b->nscenes = nscenes;
+    b->largest = 0;
+    for (const auto& x : info) b->largest = std::max(b->largest, x.nbody);
     b->hinfo = info;
     b->hplane_idx = pidx;
     b->scene_mu = false;

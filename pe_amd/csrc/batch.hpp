@@ -13,6 +13,7 @@ constexpr uint32_t kBatchMaxBodies = 4096;  // bodies per scene (LDS claim table
 constexpr uint32_t kBatchMaxPlanes = 16;
 constexpr uint32_t kBatchTable = 4096;      // buckets of a scene's hash grid (LDS)
 constexpr uint32_t kBatchMaxThreads = 512;
+constexpr uint32_t kBatchWideThreads = 256; // ... of the kernels that take a SIMD's whole register file
 
 // Host-computed description of one scene.
 struct SceneInfo {
@@ -60,11 +61,11 @@ struct BatchArgs {
 pehip_status check_params(const pehip_params* p, std::string& why);
 
 void launch_batch(int model, bool exact_trig, const Bodies& B, const RawContacts& R, const SolverContacts& C,
-                  const BatchArgs& A, uint32_t grid, uint32_t threads, hipStream_t s);
+                  const BatchArgs& A, uint32_t grid, uint32_t threads, bool wide, hipStream_t s);
 void launch_batch_fast(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C, const BatchArgs& A,
-                       uint32_t grid, uint32_t threads, hipStream_t s);
+                       uint32_t grid, uint32_t threads, bool wide, hipStream_t s);
 void launch_batch_exact(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C, const BatchArgs& A,
-                        uint32_t grid, uint32_t threads, hipStream_t s);
+                        uint32_t grid, uint32_t threads, bool wide, hipStream_t s);
 // queue[0] = 0, queue[1] += add_steps (a kernel, so that captured graphs hold no memset).
 void launch_batch_begin(uint32_t* queue, uint32_t add_steps, hipStream_t s);
 

@@ -27,6 +27,12 @@ namespace {
 
 constexpr uint32_t kEmptyKey = 0xFFFFFFFFu;
 constexpr double kBatchSpanFill = 0.999999;
+// LDS for the velocity corrections of the bodies (two a contact) of as many contacts as threads; for 64 threads
+// it is taken from tab's end.
+constexpr uint32_t batch_ldvw_bytes(uint32_t threads) { return 2 * threads * 6 * (uint32_t)sizeof(double); }
+constexpr uint32_t kBatchTailFree = kBatchTable - batch_ldvw_bytes(64) / 4;
+static_assert(kBatchTailFree % 2 == 0, "the corrections are aligned");
+static_assert(kBatchWideThreads == kResidentThreads, "a workgroup holds a contact a thread");
 
 // Inclusive/exclusive scan of one value per thread over the workgroup (blockDim.x a
 // multiple of 64, at most 512).  red needs 8 words.
@@ -162,7 +168,7 @@ __device__ __attribute__((noinline)) double relax_slide_lane(const SolverContact
 
 // One time step of scene sc.  Returns false (uniformly) if the scene hit an error; its
 // flags are then set and it does not advance.
-template <int MODEL, class Trig, uint32_t MAXT>
+template <int MODEL, class Trig, bool WIDE>
 __device__ bool scene_step(const Bodies& B, const RawContacts& R, const SolverContacts& C, const BatchArgs& A,
                            const SceneInfo& S, uint32_t sc, uint32_t* tab, uint32_t* coff, uint32_t* red,
                            unsigned long long* red64, uint32_t* lflag, double* ldvw) {
@@ -362,20 +368,18 @@ __device__ bool scene_step(const Bodies& B, const RawContacts& R, const SolverCo
     return false;
   }
 
-  // ---- sweeps.  Scenes of at most T contacts of a model without a search: everything on the chip, see
-  // resident.hpp.  Model 3, by at most 256 threads, in two parts a colour: every contact by one lane, except that the sliding ones go on a list (in tab: a colour's contacts share no
-  // non-fixed body, so it holds them), which the wavefronts then take one contact at a time.  A colour of a
-  // scene holds few contacts, of which up to a third slide; a lane's search takes 12.6k cycles a pass however
-  // few of its wavefront's lanes search, a wavefront's 3.0k to 3.7k.  (Measured for this model too: the
-  // contacts on the chip, each wavefront relaxing its own sliding ones: 100 against 89 ms for ten steps of
-  // 640 scenes of 50 to 2,000 spheres, because the sliding contacts of a colour, five on average, fall
-  // unevenly on the wavefronts.)  Ten steps of 1,500 scenes of 40 to 100 spheres: 37 ms with one lane a
-  // contact, 27 now; of 640 scenes of 50 to 2,000: 135 and 96.
-  // Model 5 stays with one lane a contact and the 512-thread kernel: its tree search takes a wavefront so long that
-  // lists made its batches up to 2.2 times slower (10 steps of 1,500 settled scenes of 200 to 600 spheres: 239 ms
-  // by lanes, 527 with lists; of 640 scenes of 50 to 2,000, still falling: 59 and 86).
-  constexpr bool kSearches = MODEL == 3 && MAXT <= 256;
-  constexpr bool kResident = MODEL != 3 && MODEL != 5 && MAXT <= kResidentThreads;
+  // ---- sweeps.  Models without a search, scenes of at most as many contacts as threads (256 at most): everything
+  // on the chip, see resident.hpp.  Model 3's WIDE kernel, in two parts a colour: every contact by one lane,
+  // except that the sliding ones go on a list (in tab: a colour's contacts share no non-fixed body, so it holds
+  // them), which the wavefronts then take one contact at a time.  A colour of a scene holds few contacts, of which
+  // up to a third slide; a lane's search takes 12.6k cycles a pass however few of its wavefront's lanes search, a
+  // wavefront's 3.0k to 3.7k.  (Measured for this model too: the contacts on the chip, each wavefront relaxing its
+  // own sliding ones: 100 against 89 ms for ten steps of 640 scenes of 50 to 2,000 spheres, because the sliding
+  // contacts of a colour, five on average, fall unevenly on the wavefronts.)  Model 5 stays with one lane a
+  // contact and the narrow kernel: its tree search takes a wavefront so long that lists made its batches up to 2.2
+  // times slower (10 steps of 1,500 settled scenes of 200 to 600 spheres: 239 ms by lanes, 527 with lists; of 640
+  // scenes of 50 to 2,000, still falling: 59 and 86).
+  constexpr bool kSearches = WIDE && MODEL == 3, kResident = MODEL != 3 && MODEL != 5;
   // Three counts in turn: the one of the colour before is cleared between this colour's first barrier,
   // when every thread has read it, and the next colour's, behind which it is used again.
   uint32_t* slide_count = red + 13;    // (the scans use the first eight words)
@@ -388,7 +392,7 @@ __device__ bool scene_step(const Bodies& B, const RawContacts& R, const SolverCo
   double last = 0;
   bool resident = false;
   if constexpr (kResident) {
-    resident = nc != 0 && nc <= T;
+    resident = nc != 0 && nc <= T && T <= kResidentThreads && (T > 64 || S.nbody <= kBatchTailFree);
     if (resident) {
       // places in LDS for the contacts' non-fixed bodies, in arrival order
       for (uint32_t i = tid; i < S.nbody; i += T) tab[i] = kNoBody;
@@ -489,14 +493,18 @@ __device__ bool scene_step(const Bodies& B, const RawContacts& R, const SolverCo
 
 }  // namespace
 
-// MAXT: the workgroups' largest size.  Up to 256 threads a wavefront has its SIMD's whole register file, and
-// without spills a search is twice as fast as within the half that 512 threads leave (89 against 160 ms for
-// ten steps of 640 scenes of 50 to 2,000 spheres).
-template <int MODEL, class Trig, uint32_t MAXT>
-__global__ void __launch_bounds__(MAXT) k_batch(Bodies B, RawContacts R, SolverContacts C, BatchArgs A) {
-  constexpr bool kResident = MODEL != 3 && MODEL != 5 && MAXT <= kResidentThreads;
-  __shared__ double ldvw[kResident ? 6 * kResidentBodies : 1];
-  __shared__ uint32_t tab[kBatchTable + 1];
+// Two kernels a model; batch_wide() in batch.hip chooses.  WIDE: workgroups of at most 256 threads, bounded for
+// them, so that a wavefront has its SIMD's whole register file and one 256-thread workgroup fills a CU; model 3's
+// search spills 16 registers instead of 186, which makes it twice as fast.  Otherwise up to 512 threads within half
+// of the file, two wavefronts a SIMD.  Corrections on the chip: 96 bytes a thread of dynamic LDS; one
+// wavefront's lie behind the bodies' places in tab (scenes of up to kBatchTailFree bodies), so that eight of
+// its workgroups still share a CU's 160 KB.
+template <int MODEL, class Trig, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? kBatchWideThreads : kBatchMaxThreads) k_batch(Bodies B, RawContacts R,
+                                                                                       SolverContacts C, BatchArgs A) {
+  extern __shared__ double dyn[];
+  __shared__ alignas(8) uint32_t tab[kBatchTable + 1];
+  double* ldvw = blockDim.x == 64 ? reinterpret_cast<double*>(tab + kBatchTailFree) : dyn;
   __shared__ uint32_t coff[kMaxColours + 1];
   __shared__ uint32_t red[16];
   __shared__ unsigned long long red64[8];
@@ -516,7 +524,7 @@ __global__ void __launch_bounds__(MAXT) k_batch(Bodies B, RawContacts R, SolverC
     __syncthreads();
     if (threadIdx.x == 0) A.out[sc].flags = 0;
     while (done < target) {
-      if (!scene_step<MODEL, Trig, MAXT>(B, R, C, A, S, sc, tab, coff, red, red64, &lflag, ldvw)) break;
+      if (!scene_step<MODEL, Trig, WIDE>(B, R, C, A, S, sc, tab, coff, red, red64, &lflag, ldvw)) break;
       ++done;
       if (threadIdx.x == 0) A.out[sc].steps = done;
     }
@@ -524,25 +532,22 @@ __global__ void __launch_bounds__(MAXT) k_batch(Bodies B, RawContacts R, SolverC
   }
 }
 
-template <class Trig, uint32_t MAXT>
-static void batch_dispatch(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C,
-                           const BatchArgs& A, uint32_t grid, uint32_t threads, hipStream_t s) {
-  const dim3 g(grid), b(threads);
-  switch (model) {
-    case 0: hipLaunchKernelGGL((k_batch<0, Trig, MAXT>), g, b, 0, s, B, R, C, A); break;
-    case 1: hipLaunchKernelGGL((k_batch<1, Trig, MAXT>), g, b, 0, s, B, R, C, A); break;
-    case 2: hipLaunchKernelGGL((k_batch<2, Trig, MAXT>), g, b, 0, s, B, R, C, A); break;
-    case 4: hipLaunchKernelGGL((k_batch<4, Trig, MAXT>), g, b, 0, s, B, R, C, A); break;
-    case 5: hipLaunchKernelGGL((k_batch<5, Trig, MAXT>), g, b, 0, s, B, R, C, A); break;
-    default: hipLaunchKernelGGL((k_batch<3, Trig, MAXT>), g, b, 0, s, B, R, C, A); break;
-  }
-}
-
 template <class Trig>
-static void batch_dispatch_threads(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C,
-                                   const BatchArgs& A, uint32_t grid, uint32_t threads, hipStream_t s) {
-  if (threads <= 256 && model != 5) batch_dispatch<Trig, 256>(model, B, R, C, A, grid, threads, s);
-  else batch_dispatch<Trig, kBatchMaxThreads>(model, B, R, C, A, grid, threads, s);
+static void batch_dispatch(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C,
+                           const BatchArgs& A, uint32_t grid, uint32_t threads, bool wide, hipStream_t s) {
+  const dim3 g(grid), b(threads);
+  const bool resident = model != 3 && model != 5 && threads > 64 && threads <= kResidentThreads;
+  const uint32_t lds = resident ? batch_ldvw_bytes(threads) : 0;
+#define PE_BATCH(model, wide) hipLaunchKernelGGL((k_batch<model, Trig, wide>), g, b, lds, s, B, R, C, A)
+  switch (model) {
+    case 0: if (wide) PE_BATCH(0, true); else PE_BATCH(0, false); break;
+    case 1: if (wide) PE_BATCH(1, true); else PE_BATCH(1, false); break;
+    case 2: if (wide) PE_BATCH(2, true); else PE_BATCH(2, false); break;
+    case 4: if (wide) PE_BATCH(4, true); else PE_BATCH(4, false); break;
+    case 5: PE_BATCH(5, false); break;
+    default: if (wide) PE_BATCH(3, true); else PE_BATCH(3, false); break;
+  }
+#undef PE_BATCH
 }
 
 }  // namespace pe_amd

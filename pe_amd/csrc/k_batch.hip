@@ -4,8 +4,8 @@
 namespace pe_amd {
 
 void launch_batch_fast(int model, const Bodies& B, const RawContacts& R, const SolverContacts& C, const BatchArgs& A,
-                      uint32_t grid, uint32_t threads, hipStream_t s) {
-  batch_dispatch_threads<TrigFast>(model, B, R, C, A, grid, threads, s);
+                      uint32_t grid, uint32_t threads, bool wide, hipStream_t s) {
+  batch_dispatch<TrigFast>(model, B, R, C, A, grid, threads, wide, s);
 }
 
 __global__ void k_batch_begin(uint32_t* queue, uint32_t add_steps) {
@@ -20,9 +20,9 @@ void launch_batch_begin(uint32_t* queue, uint32_t add_steps, hipStream_t s) {
 }
 
 void launch_batch(int model, bool exact_trig, const Bodies& B, const RawContacts& R, const SolverContacts& C,
-                  const BatchArgs& A, uint32_t grid, uint32_t threads, hipStream_t s) {
-  if (exact_trig) launch_batch_exact(model, B, R, C, A, grid, threads, s);
-  else launch_batch_fast(model, B, R, C, A, grid, threads, s);
+                  const BatchArgs& A, uint32_t grid, uint32_t threads, bool wide, hipStream_t s) {
+  if (exact_trig) launch_batch_exact(model, B, R, C, A, grid, threads, wide, s);
+  else launch_batch_fast(model, B, R, C, A, grid, threads, wide, s);
 }
 
 }  // namespace pe_amd

@@ -38,6 +38,19 @@ def stacks(contacts, model, sweeps, same=False):
                         v0=np.concatenate([np.zeros((1, 3)), v]), dt=1e-3, max_iterations=sweeps, model=model)
 
 
+def pairs(contacts, model, sweeps):
+    """Falling pairs of spheres that touch: two bodies a contact."""
+    rng = np.random.default_rng(contacts)
+    side = int(np.ceil(np.sqrt(contacts)))
+    at = np.stack([3.0 * (np.arange(contacts) % side), 3.0 * (np.arange(contacts) // side), np.full(contacts, 9.0)], axis=1)
+    pos = np.concatenate([at, at + [0.6, 0.0, 0.8 - 1e-7]])
+    v = rng.uniform(-0.3, 0.3, size=pos.shape)
+    v[contacts:] -= [0.3, 0.0, 0.4]                  # the upper one comes nearer
+    return scenes.Scene("pairs", MATERIAL, [((0, 0, 1), 0.0, 0)], pos, np.full(len(pos), 0.5),
+                        np.zeros(len(pos), np.uint32), v0=np.concatenate([np.zeros((1, 3)), v]), dt=1e-3,
+                        max_iterations=sweeps, model=model)
+
+
 def step(scene, schedule, abort=0.0):
     w = World(device=0)
     scene.to_world(w)
@@ -64,6 +77,17 @@ def test_automatic_choice_equals_colour_launches(contacts, model, abort):
     a, b = step(sc, 0, abort), step(sc, 1, abort)
     assert a[2]["num_contacts"] == contacts
     assert (a[2]["schedule_used"] == 3) == (contacts <= 768)
+    same(a, b)
+
+
+# two bodies a contact fill the table of the bodies' places
+@pytest.mark.parametrize("contacts", [256, 768])
+@pytest.mark.parametrize("model", [0, 1, 2, 4])
+def test_pairs_fill_the_workgroup(contacts, model):
+    sc = pairs(contacts, model, 20)
+    a, b = step(sc, 0), step(sc, 1)
+    assert a[2]["num_contacts"] == contacts and a[2]["schedule_used"] == 3
+    assert np.abs(a[1]).max() > 0
     same(a, b)
 
 
