@@ -421,8 +421,9 @@ void adj_init(uint32_t n, const uint8_t* fixed, const double* xbar, const double
               double* alpha, hipStream_t s);
 void adj_sweep(const AdjTape& T, uint32_t begin, uint32_t end, const double* pk, double* alpha, double* lambda,
                unsigned long long* delta, hipStream_t s);
-// All sweeps in one workgroup (see k_adj_block), for up to kAdjBlockContacts contacts; false beyond.
-constexpr uint32_t kAdjHeldContacts = 512, kAdjHeldBodies = 2048, kAdjBlockContacts = 2048;
+// All sweeps in one workgroup (see k_adj_block), for up to kAdjBlockContacts contacts, kAdjBlockColour a colour on
+// average; false beyond.
+constexpr uint32_t kAdjHeldContacts = 512, kAdjHeldBodies = 2048, kAdjBlockContacts = 2048, kAdjBlockColour = 550;
 bool adj_block(const AdjTape& T, const struct ColourOffsets& O, uint32_t n, const double* pk, double* alpha,
                double* lambda, uint32_t sweeps, double tol, unsigned long long* out, hipStream_t s);
 void adj_assemble(const AdjTape& T, const double* jac, const double* alpha, const double* lambda, double* xbar,

@@ -210,7 +210,7 @@ __global__ void k_adj_sweep(AdjTape T, uint32_t begin, uint32_t end, const doubl
 }
 
 // All sweeps of a step in one workgroup, a barrier between colours (the contacts of one share no non-fixed
-// body, so these are the colour launches' updates, bit for bit) and the host's test for the end -- the
+// body, so these are the colour launches' updates in their order) and the host's test for the end -- the
 // change of every eighth sweep and of the last against tol, if tol > 0.  out[0]: sweeps done, out[1]: the
 // change last looked at (the last sweep's without tol).
 //
@@ -219,6 +219,10 @@ __global__ void k_adj_sweep(AdjTape T, uint32_t begin, uint32_t end, const doubl
 // L2.  576 contacts in 8 colours, 2,000 sweeps: about 45 ms from L2 against 130 by colour launches (1,024
 // threads, whose 128 registers do not hold a contact's fields at once: 117); up to 180 contacts in 2 or 3
 // colours, held: 2.2 us a sweep against 12.
+//   From L2 a colour costs about 3.6 us and 14 ns a contact, a colour launch 11 to 13 us: kAdjBlockColour contacts a
+// colour on average.  Reverse pass of two steps of 400 sweeps, one workgroup against colour launches: blocks of
+// 931 contacts in 8 colours 38 against 66 ms, 1,408 in 9: 42 and 71, 2,025 in 8: 50 and 74; in 2 colours 1,000
+// contacts 16.5 and 20.7, 1,100: 19.7 and 20.7, 1,200: 21.0 and 20.5, 2,000: 28 and 21.
 template <bool HOLD, uint32_t THREADS>
 __global__ void __launch_bounds__(THREADS) k_adj_block(AdjTape T, ColourOffsets O, uint32_t n, const double* pk,
                                                        double* alpha, double* lambda, uint32_t sweeps, double tol,
@@ -389,7 +393,7 @@ bool adj_block(const AdjTape& T, const ColourOffsets& O, uint32_t n, const doubl
   if (T.nc <= kAdjHeldContacts && n <= kAdjHeldBodies)
     hipLaunchKernelGGL((k_adj_block<true, kAdjHeldContacts>), dim3(1), dim3(kAdjHeldContacts), 0, s, T, O, n, pk,
                        alpha, lambda, sweeps, tol, out);
-  else if (T.nc <= kAdjBlockContacts)
+  else if (T.nc <= kAdjBlockContacts && T.nc <= kAdjBlockColour * O.ncol)
     hipLaunchKernelGGL((k_adj_block<false, 512>), dim3(1), dim3(512), 0, s, T, O, n, pk, alpha, lambda, sweeps, tol,
                        out);
   else return false;

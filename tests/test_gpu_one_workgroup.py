@@ -122,8 +122,8 @@ def gradient(contacts, like=None):
     return g, pairs
 
 
-# held in registers (512), from L2 (2,048), colour launches
-@pytest.mark.parametrize("contacts", [510, 512, 514, 2048, 2050])
+# held in registers (up to 512), from L2 (up to 550 a colour: the stacks have two), colour launches
+@pytest.mark.parametrize("contacts", [510, 512, 514, 1100, 1102, 2048, 2050])
 def test_adjoint_of_many_stacks_is_each_stacks_own(contacts):
     (gx, gv, gw, gmu), _ = gradient(2, like=contacts)
     (hx, hv, hw, hmu), pairs = gradient(contacts)
@@ -134,3 +134,46 @@ def test_adjoint_of_many_stacks_is_each_stacks_own(contacts):
             # overlaps of 1e-7, and both runs converge to 1e-13
             assert np.max(np.abs(rows - g[1 + k])) <= 1e-6 * max(1.0, np.max(np.abs(g)))
     assert abs(hmu - pairs * gmu) <= 1e-6 * pairs * max(1.0, abs(gmu))
+
+
+def towers(count, floating=0):
+    """Towers of three spheres that lean, each with a floor contact, all alike, and free spheres above them."""
+    side = int(np.ceil(np.sqrt(count)))
+    at = 3.0 * np.stack([np.arange(count) % side, np.arange(count) // side], axis=1) + 1.0
+    step_up = np.sqrt(1.0 - 0.0125) - 3e-7
+    pos = np.concatenate([np.concatenate([at + [0.1 * k, 0.05 * k], np.full((count, 1), 0.5 - 1e-7 + k * step_up)], axis=1)
+                          for k in range(3)])
+    v = np.repeat(np.random.default_rng(5).uniform(-0.05, 0.05, size=(3, 3)), count, axis=0)
+    v[:, 2] = -0.05
+    k = np.arange(floating)
+    free = np.stack([2.0 * (k % 64), 2.0 * (k // 64), np.full(floating, 20.0)], axis=1)
+    pos, v = np.concatenate([pos, free]), np.concatenate([v, np.zeros((floating, 3))])
+    return scenes.Scene("towers", MATERIAL, [((0, 0, 1), 0.0, 0)], pos, np.full(len(pos), 0.5),
+                        np.zeros(len(pos), np.uint32), v0=np.concatenate([np.zeros((1, 3)), v]), dt=1e-3,
+                        max_iterations=400, model=1)
+
+
+def tower_gradient(count, floating=0):
+    sc = towers(count, floating)
+    run = DifferentiableRun(sc, 3, checkpoint_every=3, max_iterations=2000, abort_threshold=1e-13, adjoint_sweeps=2000,
+                            adjoint_tol=1e-13)
+    run.forward(sc.v0[1:], 0.4)
+    weight = np.zeros((len(sc.v0), 3))
+    for k, w in enumerate(([1.0, -0.5, 0.25], [-0.75, 0.5, 1.0], [0.5, 0.75, -1.0])):
+        weight[1 + k * count:1 + (k + 1) * count] = w
+    g = run.backward(weight)
+    assert run.last_stats["max_contacts"] == 3 * count
+    run.close()
+    return [x[1:1 + 3 * count] for x in g[:3]], g[3]
+
+
+# coupled contacts: held, from L2 for the bodies' sake (more than 2,048) or the contacts', colour launches
+@pytest.mark.parametrize("count,floating", [(1, 2044), (1, 2045), (170, 0), (171, 0), (366, 0), (700, 0)])
+def test_adjoint_of_towers_is_each_towers_own(count, floating):
+    g, gmu = tower_gradient(1)
+    h, hmu = tower_gradient(count, floating)
+    for a, b in zip(g, h):
+        for k in range(3):
+            # as above: places of 1e-14 against overlaps of 1e-7, through three contacts one above the other
+            assert np.max(np.abs(b[k * count:(k + 1) * count] - a[k])) <= 4e-6 * max(1.0, np.max(np.abs(a)))
+    assert abs(hmu - count * gmu) <= 4e-6 * count * max(1.0, abs(gmu))
