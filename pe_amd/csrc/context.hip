@@ -19,7 +19,10 @@ namespace {
 
 const char* kVersion = "pe_hip 0.1.0 (gfx950)";
 // Automatic schedule: dataflow sweeps up to this many contacts (above it a colour holds enough
-// contacts to fill the device and the colour launches are throughput-bound, not latency-bound).
+// contacts to fill the device and the colour launches are throughput-bound, not latency-bound).  30 sweeps
+// of model 3 on lattices of touching spheres (9 to 10 colours), dataflow against colour launches: 43,110 contacts
+// 5.6 and 8.7 ms, 61,414: 7.9 and 8.7, 85,802: 11.0 and 9.2, 137,474: 17.4 and 11.0.  (Model 5 crosses at about
+// 100,000, 6.9 and 7.7 ms at 85,802; model 1 at about 50,000, 5.0 and 4.0 ms at 61,414.)
 constexpr uint32_t kDataflowMaxContacts = 65536;
 // Polls (each with a short sleep) before a waiting wavefront gives up: seconds, far above any
 // legitimate wait.
@@ -27,11 +30,18 @@ constexpr uint32_t kDataflowSpinLimit = 1u << 22;
 // With an abort threshold the host reads the device's stop flag once per this many sweeps.
 constexpr uint32_t kAbortPoll = 32;
 // Automatic schedule: one workgroup runs all sweeps of a step while it holds all the contacts on the chip
-// (models without a search).  A colour costs it 1 to 2 us; an update costs the dataflow sweeps about 4 us, and
-// so does a colour launch, the choice with an abort threshold.  50 sweeps of model 1, one workgroup against
-// dataflow: 0.22 against 0.41 ms (18 contacts), 0.22 against 0.65 (100), 0.23 against 0.63 (194), 0.43 against
-// 0.66 (281), 0.48 against 0.70 (408).  (Models with a search: a workgroup relaxes four sliding contacts at a
-// time; model 3 0.44 against 0.50 (18), 0.96 against 0.79 (39), 3.2 against 1.0 (144).)
+// (models without a search).  A colour costs it 0.8 to 1.3 us with up to 256 contacts, whose bodies' records it
+// holds too, and 1.3 to 2.6 us beyond (3 to 5 us for colours of 400); an update costs the dataflow sweeps about 4 us,
+// and a colour launch, the choice with an abort threshold, 11 us with its gap.  50 sweeps, one workgroup against
+// dataflow (without a threshold) and against colour launches (with one), in ms:
+//   contacts (colours)         60 (2)      256 (2)     480 (8)     672 (8)     768 (7)     768 (2)
+//   model 1   dataflow      0.13  0.54  0.13  0.69  0.80  2.04  0.91  2.03  0.90  2.01  0.46  0.68
+//             launches      0.17  1.31  0.17  1.33  0.94  4.89  0.98  4.94  0.95  4.47  0.53  1.50
+//   model 0   dataflow      0.08  0.52  0.09  0.68  0.45  2.19  0.52  2.16  0.52  2.14  0.31  0.67
+//   model 2   dataflow      0.11  0.55  0.11  0.71  0.62  2.29  0.70  2.25  0.67  2.22  0.38  0.70
+//   model 4   dataflow      0.11  0.54  0.12  0.73  0.55  2.30  0.63  2.26  0.61  2.23  0.35  0.71
+// It still wins at all it can hold.  (Models with a search: a workgroup relaxes four sliding contacts at a
+// time; model 3 0.44 against 0.50 (18 contacts), 0.96 against 0.79 (39), 3.2 against 1.0 (144).)
 constexpr uint32_t kSingleBlockMaxContacts = kResidentWide;
 
 bool choose_single_block(const pehip_params& P, uint32_t nc) {

@@ -1069,7 +1069,9 @@ struct TripleNode {
 // below); otherwise three lanes a triple.  rights: per triple j < NT - 1 the lanes whose code has bit j
 // set.  In assembly: the lanes that drop out are known, so that the execution mask is shifted (a compare
 // and a branch per advance cost 40 cycles), and the selects of all 22 instructions of an advance take
-// their masks from scalar registers.
+// their masks from scalar registers.  All 64 lanes have to be active when a walk (these and golden_walk) is
+// entered: shifting a partial mask would leave out lanes that advance and switch on ones that do not, and no
+// outcome check sees it.  Searches with SPEC 6 are called by whole wavefronts on one contact only.
 #define PE_TRIPLE_ADVANCE(shift, lm, rm)                                                                     \
   "s_lshl_b64 exec, exec, " shift "\n\t"                                                                     \
   "v_add_f64 v[8:9], v[4:5], -v[6:7]\n\t"                                                                    \

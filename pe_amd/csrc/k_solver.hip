@@ -440,16 +440,10 @@ __device__ __forceinline__ bool wait_count(const uint32_t* ctr, uint32_t target,
   }
 }
 
-// A contact's fields held in registers (the impulse excluded: it is loaded after the wait).
-struct PrefetchedFields {
-  double v[CF_COUNT];
-  __device__ __forceinline__ double operator()(int k) const { return v[k]; }
-};
-
 // relax_contact<..., COHERENT = true> with the read-only inputs already loaded: the velocity
 // corrections and the impulse by agent-scope loads, the new ones stored by lane 0 likewise.
 template <int MODEL, class Trig, int SPEC>
-__device__ __forceinline__ double relax_coherent(const SolverContacts& C, uint32_t i, const PrefetchedFields& cf,
+__device__ __forceinline__ double relax_coherent(const SolverContacts& C, uint32_t i, const HeldFields& cf,
                                                  const RelaxBody& B1, const RelaxBody& B2, uint32_t i1,
                                                  uint32_t i2, bool fx1, bool fx2, double* dvw, int maxSub) {
   const size_t cap = C.cap;
@@ -523,7 +517,7 @@ __global__ void __launch_bounds__(256) k_sweep_dataflow(SolverContacts C, uint32
     // The relaxation's read-only inputs -- the contact record and the bodies' records -- are
     // loaded before the wait, whose latency they then overlap; only the velocity corrections and
     // the impulse, which earlier items write, are loaded after it.
-    PrefetchedFields cf;
+    HeldFields cf;
 #pragma unroll
     for (int k = 0; k < CF_P; ++k) cf.v[k] = C.f[(size_t)k * C.cap + s];
 #pragma unroll
@@ -559,12 +553,13 @@ __global__ void __launch_bounds__(256) k_sweep_dataflow(SolverContacts C, uint32
 }
 
 // Lanes per contact.  A wavefront issues one instruction every four cycles whatever its lanes
-// do, so a lone contact's relaxation costs its instruction count; the speculated search with a
-// whole wavefront per contact (SPEC 6) cuts the sequential sin/cos evaluations of a pass from 20
-// to 4 rounds and measures 1.2x (device libm) to 2.8x (correctly rounded trig) faster per sliding
-// contact than one lane per contact.  Colours are small in the latency-bound regime, so the
-// largest group (64, 16, 4, 1) with which every wavefront of the colour is resident at once wins;
-// big colours fall back to more contacts per wavefront (occupancy queried once).
+// do, so a lone contact's relaxation costs its instruction count: a pass of model 3's search 12.6k cycles
+// by one lane (20 sequential sin/cos evaluations), 3.0k to 3.7k by a whole wavefront (SPEC 6, golden_circle;
+// model 5 and SPEC 2 and 4 search in tree rounds, model 5's of 6.6k cycles by a wavefront).  Colours
+// are small in the latency-bound regime, so the largest group (64, 16, 4, 1) with which every wavefront of the
+// colour is resident at once wins; big colours fall back to more contacts per wavefront (occupancy queried
+// once).  Colours of a lattice of 60,000 touching spheres: 10 us (SPEC 6), 21 (SPEC 4), 34 (SPEC 2), 47 (one lane,
+// 18,000 contacts and more).  The sizes at which the groups change were set with the tree search for SPEC 6 too.
 template <int MODEL, class Trig, int SPEC>
 static uint64_t resident_lanes(uint32_t ncu) {
   static int blocks = -1;
