@@ -216,7 +216,7 @@ __global__ void k_adj_sweep(AdjTape T, uint32_t begin, uint32_t end, const doubl
 //
 // What bounds it is the latency of a colour.  HOLD: one contact a thread with its 81 fields in registers for
 // all sweeps and the adjoints of all bodies in LDS (kAdjHeldBodies); otherwise fields and adjoints come from
-// L2.  576 contacts in 8 colours, 2,000 sweeps: about 45 ms from L2 against 130 by colour launches (1,024
+// L2.  576 contacts in 8 colours, 2,000 sweeps: 45 to 50 ms from L2 against 130 by colour launches (1,024
 // threads, whose 128 registers do not hold a contact's fields at once: 117); up to 180 contacts in 2 or 3
 // colours, held: 2.2 us a sweep against 12.
 //   From L2 a colour costs about 3.6 us and 14 ns a contact, a colour launch 11 to 13 us: kAdjBlockColour contacts a
