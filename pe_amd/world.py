@@ -143,6 +143,8 @@ class World:
         self._m_uid = []
         self._u_mass = {}        # union body index -> total mass (Union::getMass)
         self._arrays = None      # host SoA snapshot (numpy) when built
+        self._handed_out = False # host_arrays() returned that dict: its arrays may be anyone's
+        self._own_state = False  # its state arrays are setState's copies, which nobody else has seen
         self._ctx = None
         self._bodies_dirty = True
         self._params_dirty = True
@@ -284,6 +286,7 @@ class World:
             self._I, self._Iinv, self._normal, self._d = list(a["I"]), list(a["Iinv"]), list(a["normal"]), list(a["d"])
             self._uid = list(a["uid"]) if "uid" in a else [0] * len(self._shape)
             self._arrays = None
+            self._handed_out = self._own_state = False
 
     def _add(self, shape, mat, fixed, param, pos, q, inv_mass, I, Iinv, normal, d, uid=0):
         self._materialise_lists()
@@ -567,6 +570,11 @@ class World:
 
     def host_arrays(self):
         """Body arrays (numpy SoA) in body order."""
+        a = self._host_arrays()
+        self._handed_out, self._own_state = True, False
+        return a
+
+    def _host_arrays(self):
         if self._arrays is None:
             n = len(self._shape)
             self._arrays = {
@@ -612,7 +620,7 @@ class World:
             check(L.pehip_set_params(self._ctx, ctypes.byref(p)), self._ctx)
             self._params_dirty = False
         if self._bodies_dirty:
-            a = self.host_arrays()
+            a = self._host_arrays()
             n = len(a["shape"])
             if n == 0:
                 raise ValueError("no bodies")
@@ -724,7 +732,12 @@ class World:
         # the arrays given or of those handed out before
         if self._arrays is not None:
             for k in c:
-                self._arrays[k] = c[k].copy()
+                if self._own_state and self._arrays[k].shape == c[k].shape:
+                    # (new arrays cost page faults: 1.0 against 0.5 ms for 200,000 bodies)
+                    self._arrays[k][...] = c[k]
+                else:
+                    self._arrays[k] = c[k].copy()
+            self._own_state = not self._handed_out
         self._state_on_device = False
         if self._m_owner:
             if "mgpos" in st:                 # union members are placed as given

@@ -185,3 +185,35 @@ def test_the_state_given_is_the_hosts_where_its_members_are_refused(lib):
     equal(w.getState(), given)
     w.setState(given)                              # and a good one is taken again
     assert np.array_equal(w.members()["gpos"], given["mgpos"])
+
+
+def test_only_the_worlds_own_arrays_are_written_over(lib):
+    made = world(lib).host_arrays()
+    theirs = {k: v.copy() for k, v in made.items()}
+    w = World()
+    lib.worlds.append(w)
+    w.createMaterial("m", 1000.0, 0.0, 0.1, 0.1)
+    w.add_bodies(theirs)
+    states = [another(w, 0.25 * k) for k in range(1, 5)]
+    for st, given in states[:2]:
+        w.setState(st)
+    a = w.host_arrays()                            # from here on the arrays may be held
+    equal(a, states[1][1])
+    first = {k: a[k] for k, _ in FIELDS}
+    w.setState(states[2][0])
+    second = {k: a[k] for k, _ in FIELDS}
+    w.run(1, 1e-3)
+    w.host_arrays()
+    w.setState(states[3][0])
+    equal(a, states[3][1])
+    equal(first, states[1][1])
+    equal(second, states[2][1])
+    equal(theirs, made)                            # what the bodies were made from
+    for st, given in states:
+        equal(st, given)                           # and the states given
+    w.createSphere(9, (9.0, 9.0, 9.0), 0.5, 0)     # a new dict
+    st, given = another(w, 1.0)
+    w.setState(st)
+    w.setState(given)
+    equal(a, states[3][1])
+    equal(w.host_arrays(), given)
