@@ -192,22 +192,23 @@ static uint32_t grid_of(const pehip_batch* b, const pehip_batch_tuning& t) {
 
 // The wide kernel (see k_batch) halves the workgroups in flight.  It is taken where that costs nothing -- they
 // all fit at one wavefront a SIMD, or the largest scene takes longer than its share of the CUs' work takes them --
-// and with model 3 also for scenes of up to 100 bodies on average, whose sliding contacts it relaxes three times as
-// fast.  Model 5 gains nothing from it.  10 steps (piles), 3 steps (lattices) with 256 threads, the narrow kernel
-// against the wide one:
-//   model 3  200 scenes of 50 to 2,000 spheres    546 and 369 ms    640 of them   577 and 396
-//            1,500 settled scenes of 40 to 100    105 and 74        of 200 to 600  669 and 820
-//            1,024 lattices of 90 to 400           82 and 96
-//            5 steps of 1,100 settled scenes of 50 to 90 bodies: 47 and 30; 80 to 130: 99 and 94; 110 to 170: 136 and 145
-//            (lattices of 60 to 80 bodies, which fall apart in a few steps: 81 and 85)
-//   model 1  640 scenes of 50 to 2,000            20 and 16        1,024 lattices of 300 to 2,000   68 and 80
-//            1,500 scenes of 40 to 100            6.4 and 9.8       1,500 settled of 200 to 600     78 and 112
+// and with model 3 also for scenes of up to 200 bodies on average: it relaxes their sliding contacts three times as
+// fast, which wins as long as a scene holds up to some 110 contacts, as falling and small piles do.  Model 5 gains
+// nothing from it.  256 threads, the narrow kernel against the wide one, in ms:
+//   model 3, 10 steps of 200 scenes of 50 to 2,000 spheres: 546 and 369; of 640: 577 and 396; of 1,500 settled scenes of
+//   40 to 100: 105 and 74, of 200 to 600: 669 and 820; 3 steps of 1,024 lattices of 90 to 400: 82 and 96
+//   model 3, 5 steps of 1,100 scenes of   50 to 90    80 to 130   110 to 170   150 to 220   200 to 300   250 to 400
+//     falling (40 to 104 contacts)                     26  20      33  25       49  38       57  50       72  67
+//     settled (67 to 252 contacts)         47   30     99  94     136 145      172 190      217 242
+//   (lattices of 60 to 80 bodies, which fall apart in a few steps: 81 and 85)
+//   model 1, 10 steps of 640 scenes of 50 to 2,000: 20 and 16; 3 steps of 1,024 lattices of 300 to 2,000: 68 and 80; 10 steps
+//   of 1,500 scenes of 40 to 100: 6.4 and 9.8, of 1,500 settled of 200 to 600: 78 and 112
 static bool batch_wide(const pehip_batch* b, const pehip_batch_tuning& t) {
   const int model = b->prm.relaxation_model;
   if (t.threads > kBatchWideThreads || model == PEHIP_INELASTIC_GMD) return false;
   const uint64_t slots = (uint64_t)b->ncu * (kBatchWideThreads / t.threads);
   if (grid_of(b, t) <= slots || b->n <= slots * b->largest) return true;
-  return model == PEHIP_INELASTIC_COULOMB_DECOUPLING && b->n <= 100ull * b->nscenes;
+  return model == PEHIP_INELASTIC_COULOMB_DECOUPLING && b->n <= 200ull * b->nscenes;
 }
 
 static void enqueue_launch(pehip_batch* b, const BatchArgs& A, uint32_t add_steps) {

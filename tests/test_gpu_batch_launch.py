@@ -61,11 +61,13 @@ def test_few_scenes(model, abort):
     assert np.array_equal(first[1][:2 * len(sizes)], 2 * sizes)
 
 
-# more scenes than fit at one wavefront a SIMD, all of about the same size and of over 100 bodies
+# more scenes than fit at one wavefront a SIMD, all of about the same size and, for model 3, of over 200 bodies
 @pytest.mark.parametrize("model,threads,blocks", [(m, 256, 2) for m in range(6)] + [(1, 128, 4), (3, 128, 4), (1, 64, 8)])
 def test_many_scenes(model, threads, blocks):
     sizes = [threads - 1, threads, threads + 1]
     scenes = [stacks(n, model, 12) for n in sizes]
+    if threads == 128:
+        scenes = [floating(sc, 208) for sc in scenes]
     count = 1100 if threads == 256 else (1600 if threads == 128 else 2400)
     out = results([scenes[k % 3] for k in range(count)], model, 0.0, [(512, 2), (threads, blocks)])
     same(out)
